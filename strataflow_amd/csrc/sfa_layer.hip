@@ -24,8 +24,8 @@
 // [n_in, n_out]); expert stacks are [n_expert][n_out][n_in].
 #include <exception>
 
-#include "sfa_append.h"
 #include "sfa_layer.h"
+#include "sfa_mm.h"
 
 namespace sfa {
 
@@ -724,6 +724,145 @@ static int gemv_launch(const GemvParams &p, bool f16, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? SFA_OK : SFA_ERR_RUNTIME;
 }
 
+// ---- products of several tokens (sfa_mm.h) ---------------------------------------
+
+static bool aligned16(const void *a) { return reinterpret_cast<uintptr_t>(a) % 16 == 0; }
+
+// The matrix-core kernels take whole 256-byte blocks of 16-byte aligned rows
+// and 32-bit offsets into x and into a tile of W; a product with 64 outputs
+// or fewer keeps gemv_kernel, whose arithmetic sfa_moe_gate's equals bit for
+// bit, and so do two tokens, which it serves in one read of the weights
+// (4096 x 6144 F16: 14.4 us against 16.2; three: 20.8 against 16.6).  The rule reads only what sfa_mul_mat_vec and sfa_qkv_rope_kv_append
+// have in common (the shape, w and x), so both take the same kernel and their
+// results stay equal.
+static bool mm_ok(int64_t n_rows, int64_t n_in, int64_t n_out, const void *w, const void *x) {
+    return n_rows >= 3 && n_out > 64 && n_out % 4 == 0 && n_in % 128 == 0 && n_in < (1 << 22) &&
+           n_rows * n_in * 4 < ((int64_t)1 << 32) && aligned16(w) && aligned16(x);
+}
+
+template <typename WT, typename XT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
+static void mm_tile_launch(const MmArgs<OUT> &p, int n_tiles, hipStream_t s) {
+    constexpr int BMO = OUT == kMmGateUp ? BM / 2 : BM;
+    const int n_rb8 = ((p.n_out + BMO - 1) / BMO + 7) / 8 * 8;
+    hipLaunchKernelGGL((mm_tile_kernel<WT, XT, BM, BN, WR, WC, KS, G, S, OUT>), dim3((unsigned)(n_rb8 * n_tiles)),
+                       dim3(64 * WR * WC * KS), 0, s, p);
+}
+
+// Tiles of the dense products (us of a 4096 x 4096 / 4096 x 6144 / 4096 x
+// 32000 F16 product, each tile where it is taken and the next larger one
+// beside it): up to 16 tokens and 8192 outputs the skinny kernel (8 tokens
+// 11 / 20 / 65, 64 x 32 tiles 22 / 23 / 42); then the smallest tile that leaves no more than one
+// workgroup a CU (64 x 32, 128 tokens: 23 / 44 / 170), two (64 x 32 with half
+// the stages, 256 tokens: 38 / 70 / 279; 128 tokens 33 / 39 / 148), one
+// (128 x 64: 256 tokens 39 / 41 / 164), any (128 x 128: 512 tokens 57 / 59 /
+// 260).  A workgroup's time is its 64 stages' latency until the chip is full,
+// so more, smaller tiles win before that and larger ones after.  F32
+// products are bound by the matrix cores' f32 rate sooner: 32 x 32, 64 x 32
+// and 64 x 64.
+template <typename WT, int OUT>
+static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
+    const int n = p.n_rows;
+    auto tiles = [&](int bm, int bn) { return (int64_t)((p.n_out + bm - 1) / bm) * ((n + bn - 1) / bn); };
+    constexpr int kCus = 256;
+    if (n <= 16 && (p.n_out <= 8192 || sizeof(WT) == 4)) {
+        hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+    } else if (sizeof(WT) == 4) {
+        if (n <= 32)
+            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 2>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+        else if (tiles(32, 32) <= kCus)
+            mm_tile_launch<WT, float, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+        else if (tiles(64, 32) <= kCus)
+            mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 2>(p, (n + 31) / 32, s);
+        else
+            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 2>(p, (n + 63) / 64, s);
+    } else if (tiles(64, 32) <= kCus) {
+        mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+    } else if (tiles(64, 32) <= 2 * kCus) {
+        mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 2>(p, (n + 31) / 32, s);
+    } else if (tiles(128, 64) <= kCus) {
+        mm_tile_launch<WT, float, 128, 64, 2, 1, 4, 1, 3>(p, (n + 63) / 64, s);
+    } else {
+        mm_tile_launch<WT, float, 128, 128, 2, 2, 2, 1, 3>(p, (n + 127) / 128, s);
+    }
+}
+
+// ---- experts of several tokens -------------------------------------------------------
+
+// The experts of three or more tokens with F16 weights: the (token, slot) pairs
+// grouped by expert, so that an expert's weights are read once for all its
+// tokens (once a tile) and not once a pair.  The activations take half of the
+// caller's workspace (halves), the down product's rows and the plan the other
+// half; shapes whose rows do not fit there (n_ff < 2 n_embd), more than 256
+// experts and unaligned operands keep the one-pair kernels, as do two tokens
+// (four pairs seldom share an expert: 235 us against 261).  Tiles by the mean
+// number of pairs an expert has (us of two of eight 4096 x 14336 experts a
+// token): up to 6 the skinny kernel, bound by the weights (13 tokens: 445,
+// with 64-pair tiles 528; 32 tokens 556 against 534); to 45 tiles of 64 (180
+// tokens: 510, 128-pair tiles 524); above, tiles of 128 (256 tokens: 551
+// against 619; 512 tokens: 784, 64-pair tiles 860, 192-pair tiles 789,
+// 256-pair tiles 828).  The gate/up product fills the chip with two
+// workgroups of eight waves a CU; the down product has a third of the
+// workgroups and hides its loads with three stages of one.
+static bool moe_mm(const float *x, const float *residual, const int32_t *ids, const float *weights, const void *gate,
+                   const void *up, const void *down, int n_rows, int n_embd, int n_ff, int n_expert, int n_used,
+                   void *workspace, float *y, hipStream_t s) {
+    const int64_t n_pairs = (int64_t)n_rows * n_used;
+    if (n_rows < 3 || n_expert > kPlanMaxExperts || !mm_ok(n_pairs, n_embd, n_ff, gate, x) ||
+        !mm_ok(n_pairs, n_ff, n_embd, down, workspace) || !aligned16(up))
+        return false;
+    const int mean = (int)(n_pairs / n_expert);
+    const int tile = mean <= 6 ? 16 : mean <= 45 ? 64 : 128;
+    const int max_tiles = (int)(n_pairs / tile + (n_pairs < n_expert ? n_pairs : n_expert));
+    const size_t act_bytes = 2 * (size_t)n_pairs * n_ff, part_bytes = 4 * (size_t)n_pairs * n_embd;
+    const size_t plan_bytes = sizeof(MmPlan) + sizeof(MmExpert) * n_expert + 4 * (size_t)(max_tiles + n_pairs);
+    if (act_bytes + part_bytes + plan_bytes > sfa_moe_workspace_bytes(n_rows, n_used, n_ff)) return false;
+    uint8_t *ws = static_cast<uint8_t *>(workspace);
+    float *part = reinterpret_cast<float *>(ws + act_bytes);
+    half8 *x16 = reinterpret_cast<half8 *>(part);  // read by the gate/up product, before the down product writes part
+    MmPlan *plan = reinterpret_cast<MmPlan *>(ws + act_bytes + part_bytes);
+    const int64_t n_chunk = (int64_t)n_rows * n_embd / 8;
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1 + (unsigned)((n_chunk + kPlanThreads - 1) / kPlanThreads)),
+                       dim3(kPlanThreads), 0, s, ids, (int)n_pairs, n_expert, tile, max_tiles, plan, x, x16, n_chunk);
+    MmArgs<kMmGateUp> g{};
+    g.w = gate;
+    g.w2 = up;
+    g.x = x16;
+    g.n_rows = n_rows;
+    g.n_in = n_embd;
+    g.n_out = n_ff;
+    g.plan = plan;
+    g.n_expert = n_expert;
+    g.max_tiles = max_tiles;
+    g.n_used = n_used;
+    g.y = ws;
+    MmArgs<kMmDown> d{};
+    d.w = down;
+    d.x = ws;
+    d.n_rows = n_rows;
+    d.n_in = n_ff;
+    d.n_out = n_embd;
+    d.plan = plan;
+    d.n_expert = n_expert;
+    d.max_tiles = max_tiles;
+    d.n_used = n_used;
+    d.y = part;
+    if (tile == 16) {
+        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, kMmGateUp, 1>), dim3((n_ff + 15) / 16, max_tiles),
+                           dim3(512), 0, s, g);
+        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, kMmDown, 1>), dim3((n_embd + 15) / 16, max_tiles),
+                           dim3(512), 0, s, d);
+    } else if (tile == 64) {
+        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 3>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 3>(d, max_tiles, s);
+    } else {
+        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 2>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 128, 128, 2, 2, 2, 1, 3>(d, max_tiles, s);
+    }
+    hipLaunchKernelGGL(moe_combine_kernel, dim3((n_embd + 1023) / 1024, n_rows), dim3(256), 0, s, part, ids, weights,
+                       residual, y, n_embd, n_expert, n_used);
+    return true;
+}
+
 static bool weight_type_ok(int t) { return t == SFA_KV_F32 || t == SFA_KV_F16; }
 
 }  // namespace sfa
@@ -753,6 +892,21 @@ SFA_API int sfa_mul_mat_vec(const void *w, int32_t w_type, const float *x, const
         if (!sfa::weight_type_ok(w_type) || n_in % 8 != 0) return SFA_ERR_UNSUPPORTED;
         if ((n_rows + 7) / 8 > 65535) return SFA_ERR_UNSUPPORTED;  // token blocks on grid y
         if (n_rows == 0) return SFA_OK;
+        if (sfa::mm_ok(n_rows, n_in, n_out, w, x)) {
+            sfa::MmArgs<sfa::kMmDense> a{};
+            a.w = w;
+            a.x = x;
+            a.n_rows = n_rows;
+            a.n_in = n_in;
+            a.n_out = n_out;
+            a.residual = residual;
+            a.y = y;
+            if (w_type == SFA_KV_F16)
+                sfa::mm_launch<_Float16>(a, static_cast<hipStream_t>(stream));
+            else
+                sfa::mm_launch<float>(a, static_cast<hipStream_t>(stream));
+            return hipGetLastError() == hipSuccess ? SFA_OK : SFA_ERR_RUNTIME;
+        }
         const sfa::GemvParams p{w, x, residual, y, n_rows, n_in, n_out};
         return sfa::gemv_launch(p, w_type == SFA_KV_F16, static_cast<hipStream_t>(stream));
     } catch (...) {
@@ -864,6 +1018,24 @@ SFA_API int sfa_qkv_rope_kv_append(const sfa_kv_desc *kv, const void *w_qkv, int
         a.max_pages = max_pages;
         const dim3 grid((unsigned)(p.n_out / sfa::kLayerWaves), (unsigned)n_tok);
         const hipStream_t s = static_cast<hipStream_t>(stream);
+        if (sfa::mm_ok(n_tok, n_embd, p.n_out, w_qkv, x)) {  // sfa_mul_mat_vec's rule: the results stay equal
+            sfa::MmArgs<sfa::kMmQkv> m{};
+            m.w = w_qkv;
+            m.x = x;
+            m.n_rows = n_tok;
+            m.n_in = n_embd;
+            m.n_out = p.n_out;
+            m.q = q;
+            m.n_q = p.n_q;
+            m.theta_scale = p.theta_scale;
+            m.ap = a;
+            m.kv_type = kv->kv_type;
+            if (w_type == SFA_KV_F16)
+                sfa::mm_launch<_Float16>(m, s);
+            else
+                sfa::mm_launch<float>(m, s);
+            return hipGetLastError() == hipSuccess ? SFA_OK : SFA_ERR_RUNTIME;
+        }
         const bool f16w = w_type == SFA_KV_F16;
         if (kv->kv_type == SFA_KV_F16) {
             if (f16w) hipLaunchKernelGGL((sfa::qkv_rope_append_kernel<true, SFA_KV_F16>), grid, dim3(sfa::kQkvThreads), 0, s, p);
@@ -902,6 +1074,9 @@ SFA_API int sfa_moe_ffn(const float *x, const float *residual, const int32_t *id
                          y, n_rows, n_embd, n_ff, n_expert, n_used};
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const bool f16 = w_type == SFA_KV_F16;
+        if (f16 && sfa::moe_mm(x, residual, ids, weights, gate_exps, up_exps, down_exps, n_rows, n_embd, n_ff, n_expert,
+                               n_used, workspace, y, s))
+            return hipGetLastError() == hipSuccess ? SFA_OK : SFA_ERR_RUNTIME;
         const dim3 g1(sfa::grid_x(n_ff), n_used, n_rows);
         const dim3 g2((n_embd + sfa::kLayerWaves * sfa::kDownRows - 1) / (sfa::kLayerWaves * sfa::kDownRows), n_rows);
         if (f16)

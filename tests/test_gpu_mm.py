@@ -1,0 +1,177 @@
+"""Products of several tokens (sfa_mul_mat_vec, sfa_qkv_rope_kv_append and
+sfa_moe_ffn with three or more rows) against float64 and against the one-token
+calls, at the edges of their tiles: token counts around 16, 32, 64, 128 and
+192, output counts that end inside a tile, one k block and many, operands that
+the rule leaves to the one-token kernels.
+
+Tolerances: a sum of n products in f32, in chains of at most 8 roundings whose
+results are summed twice more, is within a few 2^-24 of the row's RMS times
+sqrt(chain length): 1e-6 of the RMS bounds 16 such roundings.  With F16
+weights an expert's activation is rounded to f16 before the down product; a
+last-ulp difference moves single roundings by 2^-11 of that activation, so
+2e-4 of the largest output there."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(gen, *shape, dtype=torch.float32, std=1.0):
+    return (torch.randn(shape, generator=gen, device="cuda") * std).to(dtype)
+
+
+def _gen(seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    return g
+
+
+def _operand(x, w):
+    return x.half().double() if w.dtype == torch.float16 else x.double()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n_rows,n_in,n_out", [
+    (3, 128, 68), (15, 256, 100), (16, 4096, 80), (17, 384, 260), (32, 512, 4096), (33, 128, 68), (65, 256, 1000),
+    (128, 2048, 2052), (129, 256, 8192), (257, 4096, 4100), (300, 384, 16384), (9, 128, 8196),
+    (5, 136, 100), (5, 128, 64), (5, 128, 70), (2, 128, 100)])  # the last four: left to the one-token kernel
+def test_products(gpu, dtype, n_rows, n_in, n_out):
+    from strataflow_amd import layer
+    g = _gen(n_rows * 31 + n_in + n_out)
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    x, r = _rand(g, n_rows, n_in), _rand(g, n_rows, n_out)
+    y = layer.mul_mat_vec(w, x)
+    ref = _operand(x, w) @ w.double().t()
+    rms = ref.square().mean().sqrt()
+    assert float((y.double() - ref).abs().max() / rms) < 3e-6
+    assert float((y.double() - ref).norm() / ref.norm()) < 2e-7
+    ones = torch.cat([layer.mul_mat_vec(w, x[t:t + 1].contiguous()) for t in (0, n_rows - 1)])
+    assert float((y[[0, n_rows - 1]] - ones).abs().max() / rms) < 3e-6
+    # the residual after the product, in place; outputs at any float address
+    buf = torch.zeros(n_rows * n_out + 1, device="cuda")
+    yr = buf[1:].view(n_rows, n_out)
+    yr.copy_(r)
+    layer.mul_mat_vec(w, x, residual=yr, out=yr)
+    assert torch.equal(yr, y + r)
+    # a one-hot activation picks a weight column exactly
+    cols = torch.randint(0, n_in, (n_rows,), generator=g, device="cuda")
+    oh = torch.zeros_like(x)
+    oh[torch.arange(n_rows, device="cuda"), cols] = 1.0
+    assert torch.equal(layer.mul_mat_vec(w, oh), w[:, cols].t().float())
+    # a token whose row is not finite leaves the others alone
+    xi = x.clone()
+    xi[n_rows // 2] = float("inf")
+    keep = [t for t in range(n_rows) if t != n_rows // 2]
+    assert torch.equal(layer.mul_mat_vec(w, xi)[keep], y[keep])
+
+
+@pytest.mark.parametrize("wdtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("kv_type", ["f16", "f32"])
+@pytest.mark.parametrize("n_tok,shape", [(2, (8, 4, 32, 256)), (3, (8, 4, 32, 256)), (16, (4, 2, 64, 384)), (40, (16, 4, 128, 512)),
+                                         (130, (8, 4, 32, 256)), (300, (32, 8, 128, 1024))])
+def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
+    """Bit for bit, with skipped tokens and a page that is not there."""
+    from strataflow_amd import layer, synth
+    from strataflow_amd.paged_kv import SFA_KV_F16, SFA_KV_F32, PagedKV
+    hq, hkv, hd, n_embd = shape
+    g = _gen(n_tok + n_embd)
+    w = _rand(g, (hq + 2 * hkv) * hd, n_embd, dtype=wdtype, std=n_embd ** -0.5)
+    x = _rand(g, n_tok, n_embd)
+    page, past = 64, 37
+    n_pages = -(-(past + n_tok) // page) + 2
+    pt = torch.from_numpy(synth.page_tables(np.random.default_rng(n_tok), [past + n_tok], page, n_pages)).cuda()
+    pt[0, -1] = n_pages + 3
+    seq = torch.zeros(n_tok, dtype=torch.int32, device="cuda")
+    pos = torch.arange(past, past + n_tok, dtype=torch.int32, device="cuda")
+    seq[1] = -1
+    kt = {"f16": SFA_KV_F16, "f32": SFA_KV_F32}[kv_type]
+    a, b = (PagedKV(1, hq, hkv, hd, kt, page, n_pages) for _ in range(2))
+    qa = a.qkv_rope_append(0, w, x, seq, pos, pt, 1e6)
+    y = layer.mul_mat_vec(w, x)
+    q, k, v = (t.contiguous() for t in y.split([hq * hd, hkv * hd, hkv * hd], 1))
+    qb = q.view(n_tok, hq, hd)
+    b.rope_append(0, qb, k.view(n_tok, hkv, hd), v.view(n_tok, hkv, hd), seq, pos, pt, 1e6)
+    assert torch.equal(qa, qb) and torch.equal(a.k, b.k) and torch.equal(a.v, b.v)
+
+
+@pytest.mark.parametrize("n_rows,n_embd,n_ff,n_expert,k", [
+    (3, 128, 384, 4, 2), (13, 256, 1024, 8, 2), (25, 256, 640, 8, 2), (70, 128, 384, 4, 3), (110, 256, 1024, 5, 2), (200, 256, 1024, 5, 2),
+    (400, 128, 512, 2, 2),
+    (6, 256, 384, 8, 2), (9, 128, 384, 300, 2), (2, 128, 384, 4, 2)])  # no room for the rows; too many experts; two tokens
+def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
+    """Against float64 and, with the same bits wherever it is run from, against
+    the tokens one at a time; ids outside the stack add nothing, one expert
+    may hold every pair, and the result may be written over the residual."""
+    from strataflow_amd import layer
+    g = _gen(n_rows + n_embd + n_ff)
+    h = torch.float16
+    gate = _rand(g, n_expert, n_ff, n_embd, dtype=h, std=n_embd ** -0.5)
+    up = _rand(g, n_expert, n_ff, n_embd, dtype=h, std=n_embd ** -0.5)
+    down = _rand(g, n_expert, n_embd, n_ff, dtype=h, std=n_ff ** -0.5)
+    x, res = _rand(g, n_rows, n_embd), _rand(g, n_rows, n_embd)
+    wts = torch.rand((n_rows, k), generator=g, device="cuda") + 0.1
+    spread = torch.rand((n_rows, n_expert), generator=g, device="cuda").argsort(-1)[:, :k].int().contiguous()
+    out_of = spread.clone()
+    out_of[::3, 0] = n_expert + 7
+    out_of[1::3, k - 1] = -1
+    one = torch.full_like(spread, n_expert - 1)
+    for ids in (spread, out_of, one, torch.full_like(spread, -1)):
+        ws = torch.full((n_rows * k * n_ff * 4,), 0xff, dtype=torch.uint8, device="cuda")  # NaNs
+        y = layer.moe_ffn(x, res, ids, wts, gate, up, down, workspace=ws)
+        ref = torch.zeros((n_rows, n_embd), dtype=torch.float64, device="cuda")
+        for e in range(n_expert):
+            t, j = torch.nonzero(ids == e, as_tuple=True)
+            if t.numel():
+                xe = x[t].half().double()
+                gv, uv = xe @ gate[e].double().t(), xe @ up[e].double().t()
+                act = (gv / (1 + torch.exp(-gv)) * uv).float().half().double()
+                ref.index_add_(0, t, (act @ down[e].double().t()) * wts[t, j].double()[:, None])
+        ref += res.double()
+        tol = 2e-4 * max(1.0, float(ref.abs().max()))
+        assert float((y.double() - ref).abs().max()) < tol
+        rows = [0, n_rows // 2, n_rows - 1]
+        single = torch.cat([layer.moe_ffn(x[t:t + 1], res[t:t + 1], ids[t:t + 1], wts[t:t + 1].contiguous(),
+                                          gate, up, down) for t in rows])
+        assert float((y[rows] - single).abs().max()) < tol
+        inplace = res.clone()
+        layer.moe_ffn(x, inplace, ids, wts, gate, up, down, out=inplace, workspace=ws)
+        assert torch.equal(inplace, y)
+
+
+def test_several_tokens_in_a_graph(gpu):
+    """The calls replay from a captured graph with the bits of eager calls."""
+    from strataflow_amd import layer
+    g = _gen(5)
+    n, n_embd, n_ff, n_expert, k = 40, 256, 1024, 8, 2
+    h = torch.float16
+    wo = _rand(g, n_embd, n_embd, dtype=h, std=0.06)
+    router = _rand(g, n_expert, n_embd, dtype=h, std=0.06)
+    gate, up = (_rand(g, n_expert, n_ff, n_embd, dtype=h, std=0.06) for _ in range(2))
+    down = _rand(g, n_expert, n_embd, n_ff, dtype=h, std=0.03)
+    norm = torch.ones(n_embd, device="cuda")
+    x = _rand(g, n, n_embd)
+    mid, cur, y = (torch.empty_like(x) for _ in range(3))
+    ids = torch.empty((n, k), dtype=torch.int32, device="cuda")
+    wts = torch.empty((n, k), device="cuda")
+    ws = torch.empty(n * k * n_ff * 4, dtype=torch.uint8, device="cuda")
+
+    def step():
+        layer.mul_mat_vec(wo, x, residual=x, out=mid)
+        layer.moe_norm_gate(mid, norm, 1e-5, router, k, out=cur, ids=ids, weights=wts)
+        layer.moe_ffn(cur, mid, ids, wts, gate, up, down, out=y, workspace=ws)
+
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for _ in range(3):
+        x.copy_(_rand(g, n, n_embd))
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = y.clone()
+        step()
+        torch.cuda.synchronize()
+        assert torch.equal(got, y)
