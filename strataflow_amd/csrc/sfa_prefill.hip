@@ -58,7 +58,6 @@ struct PrefillRows {
     bool row_ok;          // tq < T
     int q_lo, kv_hi, lo;  // block's first query position, last attended position, window start
     int tile0, tile1;     // 64-position tiles of the block's kv range (inclusive)
-    bool block_full;      // every row of the block is < T
 };
 template <int G>
 __device__ __attribute__((always_inline)) inline PrefillRows prefill_rows(const PrefillParams &p, int wave, int n) {
@@ -79,18 +78,20 @@ __device__ __attribute__((always_inline)) inline PrefillRows prefill_rows(const 
     r.lo = p.kv_lo > 0 ? p.kv_lo : 0;
     r.tile0 = r.lo / kPBN;
     r.tile1 = r.kv_hi / kPBN;
-    r.block_full = (qblk + 1) * QB <= p.T;
     return r;
 }
 
-// A tile needs masking where it meets the window start, the diagonal or rows
-// past T, or when its page was invalid (wave-uniform).
+// A tile needs masking where it meets the window start or the diagonal, or
+// when its page was invalid (wave-uniform).  Rows past T need none: a row is a
+// column of the products by itself, and theirs (Q read as zeros) are not
+// stored.  Masking every tile of a block that ends past T cost the last block
+// of a ragged chunk, the one that sets the kernel's time, 1.7x (93 tokens on
+// 8100: 228 -> 136 us).
 __device__ __attribute__((always_inline)) inline bool prefill_edge(const PrefillRows &r, int pos0, bool dead) {
-    return dead || pos0 < r.lo || pos0 + kPBN - 1 > r.q_lo || !r.block_full;
+    return dead || pos0 < r.lo || pos0 + kPBN - 1 > r.q_lo;
 }
 
-// Scores of positions outside [lo, qp] (all of them for a dead tile or a row
-// past T) -> -inf; register i of block pb is position pos0 + 32pb + 8(i/4) +
+// Scores of positions outside [lo, qp] (all of them for a dead tile) -> -inf; register i of block pb is position pos0 + 32pb + 8(i/4) +
 // 4hh + i%4.
 __device__ __attribute__((always_inline)) inline void prefill_mask(floatx16 (&s)[2], const PrefillRows &r, int pos0, int hh, bool dead) {
 #pragma unroll
@@ -98,7 +99,7 @@ __device__ __attribute__((always_inline)) inline void prefill_mask(floatx16 (&s)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int kp = pos0 + 32 * pb + 8 * (i >> 2) + 4 * hh + (i & 3);
-            s[pb][i] = (!dead && r.row_ok && kp >= r.lo && kp <= r.qp) ? s[pb][i] : -INFINITY;
+            s[pb][i] = (!dead && kp >= r.lo && kp <= r.qp) ? s[pb][i] : -INFINITY;
         }
     }
 }
@@ -841,14 +842,14 @@ __global__ __launch_bounds__(256, 2) void prefill_q8_kernel(PrefillParams p) {
         }
         // prefill_edge and prefill_mask spelled out: with the helper calls the
         // register allocator spills 296 bytes in this kernel at head_dim 128
-        const bool edge = dead || pos0 < lo || pos0 + kPBN - 1 > rows.q_lo || !rows.block_full;
+        const bool edge = dead || pos0 < lo || pos0 + kPBN - 1 > rows.q_lo;
         if (edge) {
 #pragma unroll
             for (int pb = 0; pb < 2; ++pb) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int kp = pos0 + 32 * pb + 8 * (i >> 2) + 4 * hh + (i & 3);
-                    s[pb][i] = (!dead && row_ok && kp >= lo && kp <= rows.qp) ? s[pb][i] : -INFINITY;
+                    s[pb][i] = (!dead && kp >= lo && kp <= rows.qp) ? s[pb][i] : -INFINITY;
                 }
             }
         }
