@@ -1,0 +1,55 @@
+"""The forms of sfa_attn_prefill (the split of a short chunk's history over
+waves, two groups of waves, one) against each other: a chunk whose size takes
+one form, and the same rows in chunks of 32 tokens, which take the split.  The
+split itself is compared with the oracle in the prefill sweep.
+
+Tolerance: the forms cut the positions differently, so a running maximum, and
+with it the rounding of a probability to f16 (2^-11), differs: 2^-11 of a
+probability each way, averaged over the attended positions, is under 1e-3 of
+the row.  F32 caches keep f32 throughout: the sums' order alone, 2e-6."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (heads, kv heads, head_dim), cached positions, tokens, page, first attended position
+FORMS = [
+    ((32, 32, 64), 600, 513, 64, 0),      # two groups (160 workgroups of 128 rows), g = 1, pages of one tile
+    ((64, 16, 128), 1000, 300, 64, 130),  # two groups, a window that starts inside a tile
+    ((64, 16, 128), 1003, 300, 128, 0),   # two groups, an odd number of tiles
+    ((64, 8, 64), 991, 305, 256, 0),      # two groups, g = 8
+    ((64, 16, 128), 40, 300, 256, 0),     # a short span: one group for F16
+    ((64, 16, 128), 513, 600, 64, 70),    # one group (more workgroups than CUs)
+    ((16, 4, 128), 2000, 577, 256, 0),    # the split, three waves' tiles short of a round
+    ((8, 8, 64), 0, 100, 64, 0),          # the split, fewer tiles than waves
+]
+
+
+@pytest.mark.parametrize("kv_type", ["f16", "q8_0", "f32"])
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: f"h{f[0][0]}kv{f[0][1]}d{f[0][2]}n{f[1]}t{f[2]}p{f[3]}lo{f[4]}")
+def test_forms_agree(gpu, kv_type, form):
+    from strataflow_amd import synth
+    from strataflow_amd.paged_kv import SFA_KV_F16, SFA_KV_F32, SFA_KV_Q8_0, PagedKV
+    (hq, hkv, hd), past, n_tok, page, lo = form
+    n = past + n_tok
+    n_pages = -(-n // page) + 2
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + hq)
+    kv = PagedKV(1, hq, hkv, hd, {"f16": SFA_KV_F16, "q8_0": SFA_KV_Q8_0, "f32": SFA_KV_F32}[kv_type], page, n_pages)
+    pt = torch.from_numpy(synth.page_tables(np.random.default_rng(n), [n], page, n_pages)).cuda()
+    k = torch.randn((n, hkv, hd), generator=g, device="cuda")
+    k[torch.arange(n, device="cuda") % 61 == 17] *= 5  # maxima that move late in a wave's tiles
+    v = torch.randn((n, hkv, hd), generator=g, device="cuda")
+    kv.append(0, k, v, torch.zeros(n, dtype=torch.int32, device="cuda"),
+              torch.arange(n, dtype=torch.int32, device="cuda"), pt)
+    if past > 4 * page:
+        pt[0, 2] = -1  # a page that is not there adds nothing
+    q = torch.randn((n_tok, hq, hd), generator=g, device="cuda")
+    whole = kv.prefill(0, q, pt[0], past, kv_lo=lo)
+    parts = torch.cat([kv.prefill(0, q[t:t + 32].contiguous(), pt[0], past + t, kv_lo=lo) for t in range(0, n_tok, 32)])
+    rel = float((whole.double() - parts.double()).norm() / parts.double().norm())
+    worst = float((whole - parts).abs().max())
+    assert torch.isfinite(whole).all()
+    tol = 2e-6 if kv_type == "f32" else 1e-3
+    assert rel < tol and worst < 20 * tol, (rel, worst)
