@@ -748,41 +748,46 @@ static void mm_tile_launch(const MmArgs<OUT> &p, int n_tiles, hipStream_t s) {
                        dim3(64 * WR * WC * KS), 0, s, p);
 }
 
-// Tiles of the dense products (us of a 4096 x 4096 / 4096 x 6144 / 4096 x
-// 32000 F16 product, each tile where it is taken and the next larger one
-// beside it): up to 16 tokens and 8192 outputs the skinny kernel (8 tokens
-// 11 / 20 / 65, 64 x 32 tiles 22 / 23 / 42); then the smallest tile that leaves no more than one
-// workgroup a CU (64 x 32, 128 tokens: 23 / 44 / 170), two (64 x 32 with half
-// the stages, 256 tokens: 38 / 70 / 279; 128 tokens 33 / 39 / 148), one
-// (128 x 64: 256 tokens 39 / 41 / 164), any (128 x 128: 512 tokens 57 / 59 /
-// 260).  A workgroup's time is its 64 stages' latency until the chip is full,
-// so more, smaller tiles win before that and larger ones after.  F32
-// products are bound by the matrix cores' f32 rate sooner: 32 x 32, 64 x 32
-// and 64 x 64.
+// Tiles of the dense products.  F16, us of a 4096 x 4096 / 4096 x 6144 /
+// 4096 x 32000 product with the tile taken and (the next ones): the smallest
+// tile that leaves no more than one workgroup a CU, since a workgroup's time is
+// the latency of its stages until the chip is full:
+//   skinny      16 tokens, up to 4096 outputs   13 / - / -      (32 x 32: 14 / 17 / -)
+//   32 x 32     64, 32 tokens                   17 / 18 / -     (64 x 32: 22 / 23)
+//   64 x 32     128, 64 tokens                  22 / 23 / -     (64 x 64: 29 / 30)
+//   64 x 64     256, 128 tokens                 29 / 30 / -     (128 x 64: 39 / 40; 64 x 32: 39 / 41)
+//   128 x 64    512, 256, 64 tokens             39 / 39 / 59    (64 x 64: 55 / 54 / 70)
+//   128 x 128   - , 512, 512 tokens             - / 58 / 240    (128 x 64: - / 76 / 305)
+// F32 (4096 x 4096): the matrix cores' f32 rate binds sooner: skinny to 32
+// tokens (28, 32 x 32: 36), 32 x 32 while it has two workgroups a CU (128
+// tokens: 56, 64 x 64: 82), then 64 x 64 (512 tokens: 154, 32 x 32: 199).
 template <typename WT, int OUT>
 static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
     const int n = p.n_rows;
-    auto tiles = [&](int bm, int bn) { return (int64_t)((p.n_out + bm - 1) / bm) * ((n + bn - 1) / bn); };
     constexpr int kCus = 256;
-    if (n <= 16 && (p.n_out <= 8192 || sizeof(WT) == 4)) {
-        hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
-    } else if (sizeof(WT) == 4) {
-        if (n <= 32)
+    auto tiles = [&](int bm, int bn) { return (int64_t)((p.n_out + bm - 1) / bm) * ((n + bn - 1) / bn); };
+    if constexpr (sizeof(WT) == 4) {
+        if (n <= 16)
+            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+        else if (n <= 32)
             hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 2>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+        else if (tiles(32, 32) <= 2 * kCus)
+            mm_tile_launch<WT, float, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+        else
+            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 2>(p, (n + 63) / 64, s);
+    } else {
+        if (n <= 16 && p.n_out <= 16 * kCus)
+            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
         else if (tiles(32, 32) <= kCus)
             mm_tile_launch<WT, float, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
         else if (tiles(64, 32) <= kCus)
-            mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 2>(p, (n + 31) / 32, s);
+            mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+        else if (tiles(64, 64) <= kCus)
+            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 3>(p, (n + 63) / 64, s);
+        else if (tiles(128, 64) <= kCus)
+            mm_tile_launch<WT, float, 128, 64, 2, 2, 2, 1, 4>(p, (n + 63) / 64, s);
         else
-            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 2>(p, (n + 63) / 64, s);
-    } else if (tiles(64, 32) <= kCus) {
-        mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
-    } else if (tiles(64, 32) <= 2 * kCus) {
-        mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 2>(p, (n + 31) / 32, s);
-    } else if (tiles(128, 64) <= kCus) {
-        mm_tile_launch<WT, float, 128, 64, 2, 1, 4, 1, 3>(p, (n + 63) / 64, s);
-    } else {
-        mm_tile_launch<WT, float, 128, 128, 2, 2, 2, 1, 3>(p, (n + 127) / 128, s);
+            mm_tile_launch<WT, float, 128, 128, 2, 2, 2, 1, 3>(p, (n + 127) / 128, s);
     }
 }
 
@@ -796,13 +801,12 @@ static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
 // experts and unaligned operands keep the one-pair kernels, as do two tokens
 // (four pairs seldom share an expert: 235 us against 261).  Tiles by the mean
 // number of pairs an expert has (us of two of eight 4096 x 14336 experts a
-// token): up to 6 the skinny kernel, bound by the weights (13 tokens: 445,
-// with 64-pair tiles 528; 32 tokens 556 against 534); to 45 tiles of 64 (180
-// tokens: 510, 128-pair tiles 524); above, tiles of 128 (256 tokens: 551
-// against 619; 512 tokens: 784, 64-pair tiles 860, 192-pair tiles 789,
-// 256-pair tiles 828).  The gate/up product fills the chip with two
-// workgroups of eight waves a CU; the down product has a third of the
-// workgroups and hides its loads with three stages of one.
+// token): up to 6 the skinny kernel, bound by the weights (13 tokens: 445, with
+// 64-pair tiles 528; 32 tokens 556 against 513); to 45 tiles of 64 (180
+// tokens: 548, 128-pair tiles 567); above, tiles of 128 pairs by 128 rows (256
+// tokens: 578 against 657 with 64 pairs, 655 with 256 rows) and, from 90, by
+// 256 rows, whose waves feed each operand to four products (512 tokens: 745
+// against 835).
 static bool moe_mm(const float *x, const float *residual, const int32_t *ids, const float *weights, const void *gate,
                    const void *up, const void *down, int n_rows, int n_embd, int n_ff, int n_expert, int n_used,
                    void *workspace, float *y, hipStream_t s) {
@@ -852,11 +856,14 @@ static bool moe_mm(const float *x, const float *residual, const int32_t *ids, co
         hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, kMmDown, 1>), dim3((n_embd + 15) / 16, max_tiles),
                            dim3(512), 0, s, d);
     } else if (tile == 64) {
-        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 3>(g, max_tiles, s);
-        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 3>(d, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 4>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 4>(d, max_tiles, s);
+    } else if (mean <= 90) {
+        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 4>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 4>(d, max_tiles, s);
     } else {
-        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 2>(g, max_tiles, s);
-        mm_tile_launch<_Float16, _Float16, 128, 128, 2, 2, 2, 1, 3>(d, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 256, 128, 4, 2, 1, 1, 3>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, 256, 128, 4, 2, 1, 1, 3>(d, max_tiles, s);
     }
     hipLaunchKernelGGL(moe_combine_kernel, dim3((n_embd + 1023) / 1024, n_rows), dim3(256), 0, s, part, ids, weights,
                        residual, y, n_embd, n_expert, n_used);

@@ -176,13 +176,18 @@ __device__ inline half8 mm_half8(const floatx4 a, const floatx4 b) {
 // kernels' 64 short lane sums are (k = 4096: 2.9e-7 against 0.9e-7 in f16,
 // 8.1e-7 against 1.2e-7 in f32), so the chains are cut at kMmChain additions or less
 // and their results summed this way.
-constexpr int kMmChain = 8, kMmChainF32 = 4;
+constexpr int kMmChain = 8;
 template <typename V>
 __device__ inline void mm_kahan(V &sum, V &comp, const V &v) {
     const V y = v - comp, t = sum + y;
     comp = (t - sum) - y;
     sum = t;
 }
+
+template <int N>
+struct MmInt {  // a compile-time int passed to a generic lambda
+    static constexpr int value = N;
+};
 
 // ---- up to 32 tokens ------------------------------------------------------------
 
@@ -337,6 +342,18 @@ __device__ inline void mm_sync() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
+// LDS of a tile workgroup, and the waves per SIMD that its registers leave room
+// for: as many workgroups of nw waves as the LDS of a CU holds, up to two.
+template <typename WT, typename XT>
+constexpr int mm_lds_bytes(int bm, int bn, int ks, int g, int s) {
+    const int ring = (bm * 128 + bn * (sizeof(WT) == 2 && sizeof(XT) == 4 ? 256 : 128)) * g * s, tile = ks * bm * bn * 4;
+    return ring > tile ? ring : tile;
+}
+constexpr int mm_min_waves(int nw, int lds_bytes) {
+    const int wgs = lds_bytes <= 80 * 1024 ? 2 : 1;
+    return nw * wgs >= 4 ? nw * wgs / 4 : 1;
+}
+
 // One workgroup per BM weight rows x BN tokens (gate/up: BM / 2 rows of each).
 // A stage is G slices of 128 bytes of every weight row (64 f16 or 32 f32 k)
 // and the same k of every token in LDS, S stages in a ring, loaded straight
@@ -349,10 +366,16 @@ __device__ inline void mm_sync() {
 // a slice's four k steps, so that a wave keeps a tile large enough to feed
 // each operand to several products while the workgroup stays small; the
 // groups' products meet in LDS, from where the epilogue stores whole rows.
+// The stage loop is unrolled over the ring, so that slots and chains are fixed
+// and a step's operands are read from LDS while the step before it multiplies:
+// read and used step by step, every product waited out an LDS read (moe of 512
+// tokens 58 % of the wave cycles waiting; 64 x 32 tiles 22 -> 17 us at 64
+// tokens of 4096 x 4096 as 32 x 32).
 // 1-D grid: the token tiles of one row block follow each other on one XCD
 // (XCD = L % 8), which reads its weight rows from HBM once.
 template <typename WT, typename XT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
-__global__ __launch_bounds__(64 * WR * WC * KS) void mm_tile_kernel(MmArgs<OUT> p) {
+__global__ __launch_bounds__(64 * WR * WC * KS, mm_min_waves(WR * WC * KS, mm_lds_bytes<WT, XT>(BM, BN, KS, G, S)))
+void mm_tile_kernel(MmArgs<OUT> p) {
     constexpr bool F16W = sizeof(WT) == 2;
     constexpr bool CVT = F16W && sizeof(XT) == 4;
     constexpr int NW = WR * WC * KS;                      // waves
@@ -364,7 +387,7 @@ __global__ __launch_bounds__(64 * WR * WC * KS) void mm_tile_kernel(MmArgs<OUT> 
     constexpr int NM = OUT == kMmGateUp ? 2 : 1;
     constexpr int BMO = BM / NM;                          // outputs per workgroup
     static_assert(BM % (32 * WR) == 0 && BN % (32 * WC) == 0 && 4 % KS == 0, "tile split over the waves");
-    constexpr int LDS = STAGE * G * S > KS * BM * BN * 4 ? STAGE * G * S : KS * BM * BN * 4;
+    constexpr int LDS = mm_lds_bytes<WT, XT>(BM, BN, KS, G, S);
     static_assert(LDS <= 160 * 1024, "LDS of a CU");
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
 
@@ -437,12 +460,14 @@ __global__ __launch_bounds__(64 * WR * WC * KS) void mm_tile_kernel(MmArgs<OUT> 
         }
     };
 
-    // Sums in three levels: chains of kChain additions in acc, kMmChain of
-    // those in part, those in sum.
-    constexpr int kU = 4 / KS;                        // k steps of a slice per wave
-    constexpr int kAdds = kU * (F16W ? 1 : 4);        // chained additions a slice
-    constexpr int kChain = F16W ? kMmChain : kMmChainF32;
-    constexpr int kPer = kChain / (kAdds * G) > 0 ? kChain / (kAdds * G) : 1;  // stages per chain
+    // Sums in three levels: chains of kChain k steps in acc (an F32 step is four
+    // additions), kMmChain of those in part, those in sum.
+    constexpr int kU = 4 / KS;                         // k steps of a slice per wave
+    constexpr int kSteps = G * kU;                     // .. of a stage
+    constexpr int kChain = !F16W ? 1 : KS == 1 ? kMmChain : kMmChain / 2;  // k steps per chain
+    constexpr int kPer = kChain > kSteps ? kChain / kSteps : 1;  // stages per chain
+    constexpr int kUn = S % kPer == 0 ? S : kPer % S == 0 ? kPer : S * kPer;  // stages unrolled: slot and chain are fixed in each
+    static_assert(kChain % kSteps == 0 || kSteps % kChain == 0, "chains end with a stage or within it");
     const floatx16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     floatx16 acc[FR][FC], part[FR][FC], sum[FR][FC];
@@ -450,100 +475,129 @@ __global__ __launch_bounds__(64 * WR * WC * KS) void mm_tile_kernel(MmArgs<OUT> 
     for (int a = 0; a < FR; ++a)
 #pragma unroll
         for (int b = 0; b < FC; ++b) acc[a][b] = part[a][b] = sum[a][b] = zero;
-    auto flush = [&]() {
-#pragma unroll
-        for (int a = 0; a < FR; ++a)
-#pragma unroll
-            for (int b = 0; b < FC; ++b) {
-                part[a][b] += acc[a][b];
-                acc[a][b] = zero;
-            }
-    };
-    auto flush_part = [&]() {
-#pragma unroll
-        for (int a = 0; a < FR; ++a)
-#pragma unroll
-            for (int b = 0; b < FC; ++b) {
-                sum[a][b] += part[a][b];
-                part[a][b] = zero;
-            }
-    };
 
     const int kg = wave / (WR * WC), wv = wave % (WR * WC);
     const int wr0 = (wv / WC) * FR * 32, wc = wv % WC;  // column blocks wc, wc + WC, ..
     const int n_stage = (int)(wb / (128 * G));
+    // LDS offsets of this wave's operands of k step u in a slice: rows of
+    // block 0 (the blocks' rows are 32 apart, and 32 rows keep the swizzle key)
+    int a_off[kU], b_off[kU][CVT ? 2 : 1];
+#pragma unroll
+    for (int v = 0; v < kU; ++v) {
+        const int u = KS == 1 ? v : kg * kU + v;
+        const int ar = wr0 + n, br = 32 * wc + n;
+        a_off[v] = ar * 128 + 16 * ((2 * u + hh) ^ ((ar / 2) % 8));
+        if constexpr (CVT) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) b_off[v][h] = BM * 128 + br * 256 + 16 * ((4 * u + 2 * hh + h) ^ (br % 16));
+        } else {
+            b_off[v][0] = BM * 128 + br * 128 + 16 * ((2 * u + hh) ^ ((br / 2) % 8));
+        }
+    }
+    // The stages with NC of the wave's column blocks (the others hold no token)
+    auto run = [&](auto nc) {
+        constexpr int NC = decltype(nc)::value;
+        struct Operands {
+            intx4 a[FR], b[NC][CVT ? 2 : 1];
+        };
+        auto fetch = [&](const uint8_t *st, int gv, Operands &x) {
+            const uint8_t *sl = st + (gv / kU) * STAGE;
+#pragma unroll
+            for (int i = 0; i < FR; ++i)
+                x.a[i] = *reinterpret_cast<const intx4 *>(sl + a_off[gv % kU] + 32 * 128 * i);
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+#pragma unroll
+                for (int h = 0; h < (CVT ? 2 : 1); ++h)
+                    x.b[i][h] = *reinterpret_cast<const intx4 *>(sl + b_off[gv % kU][h] + 32 * XR * WC * i);
+        };
+        int chains = 0;
+        for (int t0 = 0; t0 < n_stage; t0 += kUn) {
+#pragma unroll
+            for (int un = 0; un < kUn; ++un) {
+                const int t = t0 + un, slot = un % S;
+                if (t >= n_stage) break;
+                if (t + S - 2 < n_stage)
+                    mm_sync<(S - 2) * G * (IW + IX)>();
+                else
+                    mm_sync<0>();
+                if (t + S - 1 < n_stage) issue(t + S - 1, slot == 0 ? S - 1 : slot - 1);
+                const uint8_t *st = lds + slot * G * STAGE;
+                Operands x[2];  // the next step's are read while this one's products run
+                fetch(st, 0, x[0]);
+#pragma unroll
+                for (int gv = 0; gv < kSteps; ++gv) {
+                    if (gv + 1 < kSteps) fetch(st, gv + 1, x[(gv + 1) & 1]);
+                    const Operands &c = x[gv & 1];
+                    const bool first = kSteps >= kChain ? gv % kChain == 0 : un % kPer == 0 && gv == 0;
+#pragma unroll
+                    for (int j = 0; j < NC; ++j) {
+                        if constexpr (F16W) {
+                            half8 xh;
+                            if constexpr (CVT)
+                                xh = mm_half8(__builtin_bit_cast(floatx4, c.b[j][0]), __builtin_bit_cast(floatx4, c.b[j][CVT ? 1 : 0]));
+                            else
+                                xh = __builtin_bit_cast(half8, c.b[j][0]);
+#pragma unroll
+                            for (int i = 0; i < FR; ++i)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, c.a[i]), xh,
+                                                                                   first ? zero : acc[i][j], 0, 0, 0);
+                        } else {
+                            const floatx4 xf = __builtin_bit_cast(floatx4, c.b[j][0]);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                                for (int i = 0; i < FR; ++i)
+                                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                        __builtin_bit_cast(floatx4, c.a[i])[k], xf[k], first && k == 0 ? zero : acc[i][j], 0, 0, 0);
+                        }
+                    }
+                    const bool last = kSteps >= kChain ? gv % kChain == kChain - 1 : un % kPer == kPer - 1 && gv == kSteps - 1;
+                    if (last) {
+#pragma unroll
+                        for (int i = 0; i < FR; ++i)
+#pragma unroll
+                            for (int j = 0; j < NC; ++j) part[i][j] += acc[i][j];
+                    }
+                }
+                if (kSteps >= kChain || un % kPer == kPer - 1) {
+                    chains += kSteps >= kChain ? kSteps / kChain : 1;
+                    if (chains >= kMmChain) {
+                        chains = 0;
+#pragma unroll
+                        for (int i = 0; i < FR; ++i)
+#pragma unroll
+                            for (int j = 0; j < NC; ++j) {
+                                sum[i][j] += part[i][j];
+                                part[i][j] = zero;
+                            }
+                    }
+                }
+            }
+        }
+        if (kPer > 1 && n_stage % kPer != 0) {  // a chain that had not ended
+#pragma unroll
+            for (int i = 0; i < FR; ++i)
+#pragma unroll
+                for (int j = 0; j < NC; ++j) part[i][j] += acc[i][j];
+        }
+#pragma unroll
+        for (int i = 0; i < FR; ++i)
+#pragma unroll
+            for (int j = 0; j < NC; ++j) sum[i][j] += part[i][j];
+    };
 #pragma unroll
     for (int s = 0; s < S - 1; ++s)
         if (s < n_stage) issue(s, s);
-    int slot = 0;
-    for (int t = 0; t < n_stage; ++t) {
-        if (t + S - 2 < n_stage)
-            mm_sync<(S - 2) * G * (IW + IX)>();
+    if constexpr (kMmExperts<OUT> && FC > 1) {
+        static_assert(FC == 2, "column blocks per wave");
+        if (32 * (wc + WC) < count)
+            run(MmInt<2>{});
         else
-            mm_sync<0>();
-        if (t + S - 1 < n_stage) issue(t + S - 1, slot == 0 ? S - 1 : slot - 1);
-        const uint8_t *st = lds + slot * G * STAGE;
-        slot = slot + 1 == S ? 0 : slot + 1;
-#pragma unroll
-        for (int gv = 0; gv < G * kU; ++gv) {
-            const int v = gv % kU, u = KS == 1 ? v : kg * kU + v;
-            const uint8_t *wl = st + (gv / kU) * STAGE, *xl = wl + BM * 128;
-            intx4 a[FR], b[FC][CVT ? 2 : 1];
-#pragma unroll
-            for (int i = 0; i < FR; ++i) {
-                const int lr = wr0 + 32 * i + n;
-                a[i] = *reinterpret_cast<const intx4 *>(wl + lr * 128 + 16 * ((2 * u + hh) ^ ((lr / 2) % 8)));
-            }
-#pragma unroll
-            for (int i = 0; i < FC; ++i) {
-                const int lr = 32 * (wc + WC * i) + n;
-                if constexpr (CVT) {
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        b[i][h] = *reinterpret_cast<const intx4 *>(xl + lr * 256 + 16 * ((4 * u + 2 * hh + h) ^ (lr % 16)));
-                } else {
-                    b[i][0] = *reinterpret_cast<const intx4 *>(xl + lr * 128 + 16 * ((2 * u + hh) ^ ((lr / 2) % 8)));
-                }
-            }
-            // a chain that ends inside the stage: the next one starts from zero
-            constexpr int kStep = F16W ? kChain : kChain / 4;  // k steps per chain
-            const bool first = G * kU >= kStep && gv % kStep == 0;
-#pragma unroll
-            for (int j = 0; j < FC; ++j) {
-                if (kMmExperts<OUT> && FC > 1 && j > 0 && 32 * (wc + WC * j) >= count) continue;  // no token there
-                if constexpr (F16W) {
-                    half8 xh;
-                    if constexpr (CVT)
-                        xh = mm_half8(__builtin_bit_cast(floatx4, b[j][0]), __builtin_bit_cast(floatx4, b[j][CVT ? 1 : 0]));
-                    else
-                        xh = __builtin_bit_cast(half8, b[j][0]);
-#pragma unroll
-                    for (int i = 0; i < FR; ++i)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a[i]), xh,
-                                                                           first ? zero : acc[i][j], 0, 0, 0);
-                } else {
-                    const floatx4 xf = __builtin_bit_cast(floatx4, b[j][0]);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-#pragma unroll
-                        for (int i = 0; i < FR; ++i)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(floatx4, a[i])[k], xf[k],
-                                                                             first && k == 0 ? zero : acc[i][j], 0, 0, 0);
-                }
-            }
-            if (G * kU >= kStep && gv % kStep == kStep - 1)
-#pragma unroll
-                for (int i = 0; i < FR; ++i)
-#pragma unroll
-                    for (int j = 0; j < FC; ++j) part[i][j] += acc[i][j];
-        }
-        if constexpr (G * kAdds < kChain)
-            if (t % kPer == kPer - 1) flush();
-        constexpr int kPart = G * kAdds < kChain ? kPer * kMmChain : kMmChain * kChain / (G * kAdds);
-        if (t % kPart == kPart - 1) flush_part();
+            run(MmInt<1>{});
+    } else {
+        run(MmInt<FC>{});
     }
-    if constexpr (G * kAdds < kChain) flush();
-    flush_part();
 
     // the products into LDS, [group][token][row] with chunk c of a token at
     // c ^ (token % 8)

@@ -34,7 +34,7 @@ def _operand(x, w):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("n_rows,n_in,n_out", [
     (3, 128, 68), (15, 256, 100), (16, 4096, 80), (17, 384, 260), (32, 512, 4096), (33, 128, 68), (65, 256, 1000),
-    (128, 2048, 2052), (129, 256, 8192), (257, 4096, 4100), (300, 384, 16384), (9, 128, 8196),
+    (128, 2048, 2052), (129, 256, 8192), (257, 4096, 4100), (300, 384, 16384), (9, 128, 8196), (70, 640, 16388), (260, 384, 8196),
     (5, 136, 100), (5, 128, 64), (5, 128, 70), (2, 128, 100)])  # the last four: left to the one-token kernel
 def test_products(gpu, dtype, n_rows, n_in, n_out):
     from strataflow_amd import layer
@@ -97,7 +97,7 @@ def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
 
 @pytest.mark.parametrize("n_rows,n_embd,n_ff,n_expert,k", [
     (3, 128, 384, 4, 2), (13, 256, 1024, 8, 2), (25, 256, 640, 8, 2), (70, 128, 384, 4, 3), (110, 256, 1024, 5, 2), (200, 256, 1024, 5, 2),
-    (400, 128, 512, 2, 2),
+    (400, 128, 512, 2, 2), (150, 128, 512, 4, 2), (300, 384, 1152, 3, 2),
     (6, 256, 384, 8, 2), (9, 128, 384, 300, 2), (2, 128, 384, 4, 2)])  # no room for the rows; too many experts; two tokens
 def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
     """Against float64 and, with the same bits wherever it is run from, against
