@@ -1447,14 +1447,16 @@ __global__ __launch_bounds__(64 * kSplitWaves) void prefill_split_q8_kernel(Pref
 //   Q8_0  wg 200                 387 / 246 / 333     46 / 34 / 38
 //   Q8_0  wg 376                   - / 465 / 453      - / 57 / 70
 // So the split up to half the CUs and two groups up to all of them; short F16
-// spans above a quarter of the CUs stay with one group.
+// spans above a quarter of the CUs stay with one group, and so do the shortest
+// of all, where nothing is gained (93 tokens alone: 10 us against 12) and one
+// group's rounding is what a short prompt's results have been.
 template <int HD, int G>
 static void launch_prefill(const PrefillParams &p, int kv_type, hipStream_t s) {
     constexpr int kCus = 256;
     const int64_t wg = (int64_t)p.n_qblk * p.n_head_kv;
     const int span = p.q_pos0 + p.T - (p.kv_lo > 0 ? p.kv_lo : 0);
-    const bool f16 = kv_type == SFA_KV_F16, long_span = !f16 || span >= 1024;
-    if (kv_type == SFA_KV_F32 || wg <= kCus / 4 || (wg <= kCus / 2 && long_span)) {
+    const bool long_span = span >= (kv_type == SFA_KV_F16 ? 1024 : 512);
+    if (kv_type == SFA_KV_F32 || (wg <= kCus / 4 && span >= 512) || (wg <= kCus / 2 && long_span)) {
         PrefillParams ps = p;
         ps.n_qblk = (p.T + 32 / G - 1) / (32 / G);
         const dim3 grid(ps.n_qblk * p.n_head_kv);
