@@ -162,6 +162,13 @@ def check(status: int, what: str) -> None:
         raise SfaError(status, what)
 
 
+def current_stream() -> int:
+    """torch.cuda.current_stream().cuda_stream without building the Stream
+    object: 0.3 us of a call instead of 2.9, where a launch costs 3."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
 # ---- libsfa_host.so (include/sfa_pager.h) -----------------------------------
 
 HOST_LIB_PATH = Path(__file__).resolve().parent / "libsfa_host.so"

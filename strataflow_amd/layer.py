@@ -19,7 +19,7 @@ __all__ = ["rms_norm", "mul_mat_vec", "moe_route", "moe_gate", "moe_norm_gate", 
 
 def _stream(stream) -> int:
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return _lib.current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 

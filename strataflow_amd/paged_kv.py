@@ -36,7 +36,7 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 def _stream(stream) -> int:
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return _lib.current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 

@@ -21,7 +21,7 @@ __all__ = ["KvPager", "SFA_ATTEND_LOSSLESS", "SFA_ATTEND_WINDOW", "SFA_KV_F32", 
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _lib.current_stream()
 
 
 class KvPager:

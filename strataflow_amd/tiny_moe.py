@@ -241,24 +241,47 @@ class TinyMoeGpu(TinyMoe):
         rng = np.random.default_rng(seed)
         self.pt = torch.from_numpy(synth.page_tables(rng, [n_ctx], cfg.page_size, n_pages, max_pages)).to(device)
         self._moe_ws = None
+        # positions 0 .. n_ctx and zeros on the device: a call's pos, seq and
+        # seq_len are slices of them, not three small copies
+        self._pos = torch.arange(n_ctx + 1, dtype=torch.int32, device=device)
+        self._zero = torch.zeros(n_ctx, dtype=torch.int32, device=device)
+        # the rows of a decode step (a forward of one token ends before the
+        # next one starts: its logits have been copied to the host)
+        D, k = cfg.n_embd, cfg.n_expert_used
+
+        def buf(*shape, dtype=torch.float32):
+            return torch.empty(shape, dtype=dtype, device=device)
+
+        self._one = dict(cur=buf(1, D), q=buf(1, cfg.n_head, cfg.head_dim), attn=buf(1, cfg.n_head * cfg.head_dim),
+                         mid=buf(1, D), normed=buf(1, D), ids=buf(1, k, dtype=torch.int32), wts=buf(1, k), x=buf(1, D),
+                         logits=buf(1, cfg.n_vocab))
 
     def forward(self, tokens, pos0: int) -> np.ndarray:
         from . import layer as ops
         from .paged_kv import SFA_KV_F16, SFA_KV_F32
         torch, cfg = self.torch, self.cfg
         dev = self.device
-        tok = torch.as_tensor(np.asarray(tokens, np.int64), device=dev)
-        T = int(tok.numel())
+        ids_np = np.asarray(tokens, np.int64)
+        T = ids_np.size
         Hq, Hkv, hd = cfg.n_head, cfg.n_head_kv, cfg.head_dim
-        pos = torch.arange(pos0, pos0 + T, dtype=torch.int32, device=dev)
-        seq = torch.zeros(T, dtype=torch.int32, device=dev)
-        sl = torch.tensor([pos0 + T], dtype=torch.int32, device=dev)
-        x = self.embd.index_select(0, tok)                                  # get_rows (engine.cpp:2712)
+        if 0 <= pos0 and pos0 + T <= self.n_ctx:
+            pos, seq, sl = self._pos[pos0:pos0 + T], self._zero[:T], self._pos[pos0 + T:pos0 + T + 1]
+        else:
+            pos = torch.arange(pos0, pos0 + T, dtype=torch.int32, device=dev)
+            seq = torch.zeros(T, dtype=torch.int32, device=dev)
+            sl = torch.tensor([pos0 + T], dtype=torch.int32, device=dev)
+        one = self._one if T == 1 else {}
+        row = int(ids_np.reshape(-1)[0]) if T == 1 else -1
+        if 0 <= row < cfg.n_vocab and ids_np.ndim <= 1:                     # get_rows (engine.cpp:2712)
+            x = self.embd[row:row + 1]
+        else:
+            x = self.embd.index_select(0, torch.as_tensor(ids_np, device=dev))
         for il, L in enumerate(self.layers):
-            cur = ops.rms_norm(x, L["attn_norm"], cfg.rms_eps)
+            cur = ops.rms_norm(x, L["attn_norm"], cfg.rms_eps, out=one.get("cur"))
             if self.kv.kv_type in (SFA_KV_F16, SFA_KV_F32):
                 # the product, RoPE and the append in one launch
-                q = self.kv.qkv_rope_append(il, L["wqkv"], cur, seq, pos, self.pt, cfg.freq_base)
+                q = self.kv.qkv_rope_append(il, L["wqkv"], cur, seq, pos, self.pt, cfg.freq_base,
+                                            q=one.get("q"))
             else:  # Q8_0: a block spans 16 RoPE pairs, so the product and the append are separate
                 qkv = ops.mul_mat_vec(L["wqkv"], cur)
                 q = qkv[:, :Hq * hd].contiguous().view(T, Hq, hd)
@@ -266,16 +289,17 @@ class TinyMoeGpu(TinyMoe):
                 v = qkv[:, (Hq + Hkv) * hd:].contiguous().view(T, Hkv, hd)
                 self.kv.rope_append(il, q, k, v, seq, pos, self.pt, cfg.freq_base)
             if T == 1:
-                attn = self.kv.decode(il, q, self.pt, sl, self.n_ctx)
+                attn = self.kv.decode(il, q, self.pt, sl, self.n_ctx, out=one["attn"])
             else:
                 attn = self.kv.prefill(il, q, self.pt[0], pos0)
-            ffn_inp = ops.mul_mat_vec(L["wo"], attn, residual=x)
+            ffn_inp = ops.mul_mat_vec(L["wo"], attn, residual=x, out=one.get("mid"))
             cur, ids, wts = ops.moe_norm_gate(ffn_inp, L["ffn_norm"], cfg.rms_eps, L["gate_inp"],
-                                              cfg.n_expert_used)
+                                              cfg.n_expert_used, out=one.get("normed"), ids=one.get("ids"),
+                                              weights=one.get("wts"))
             need = T * cfg.n_expert_used * cfg.n_ff * 4
             if self._moe_ws is None or self._moe_ws.numel() < need:
                 self._moe_ws = torch.empty(need, dtype=torch.uint8, device=dev)
             x = ops.moe_ffn(cur, ffn_inp, ids, wts, L["gate_exps"], L["up_exps"], L["down_exps"],
-                            workspace=self._moe_ws)
-        h = ops.rms_norm(x[-1:].contiguous(), self.output_norm, cfg.rms_eps)
-        return ops.mul_mat_vec(self.output, h)[0].cpu().numpy()
+                            out=one.get("x"), workspace=self._moe_ws)
+        h = ops.rms_norm(x[-1:].contiguous(), self.output_norm, cfg.rms_eps, out=one.get("cur"))
+        return ops.mul_mat_vec(self.output, h, out=one.get("logits"))[0].cpu().numpy()
