@@ -405,8 +405,8 @@ def prefill_bench(torch, steps: int, warmup: int, seed: int, kv_type: int = 1, c
     res.update(with_traffic({"bound": "mfma", "achieved": round(tflops, 1),
                              "peak": peak, "unit": "TFLOP/s",
                              "frac": round(tflops / peak, 4), "traffic": None,
-                             "kernel": {0: "prefill_f32_kernel<128,4>", 1: "prefill_f16_kernel<128,4>",
-                                        8: "prefill_q8_kernel<128,4>"}[kv_type],
+                             "kernel": {0: "prefill_f32_kernel<128,4>", 1: "prefill_f16_kernel<128,4,1>",
+                                        8: "prefill_q8_kernel<128,4,1>"}[kv_type],
                              "flop_per_launch": flops},
                             {1: "prefill_2048_on_2048", 0: "prefill_f32_2048_on_2048",
                              8: "prefill_q8_0_2048_on_2048"}[kv_type]))

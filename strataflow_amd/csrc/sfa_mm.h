@@ -5,7 +5,8 @@
 //
 // Two kernels share one description of the work (MmArgs) and one epilogue
 // (mm_emit):
-//   mm_skinny_kernel  up to 32 tokens: bound by the read of the weights
+//   mm_skinny_kernel  few tokens (16; F32 weights 32): bound by the read of the
+//                     weights
 //   mm_tile_kernel    more tokens: 128-byte k slices of W and x through LDS
 // Both take the MFMA A operand from W (rows = outputs) and B from x (columns =
 // tokens), so a lane's accumulator holds four consecutive outputs of one
@@ -17,7 +18,6 @@
 
 namespace sfa {
 
-typedef float floatx4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // outputs and residuals: any float address
 typedef _Float16 half4_a2 __attribute__((ext_vector_type(4), aligned(2)));  // cache rows: any half address
 
 // What becomes of the products.
@@ -189,7 +189,7 @@ struct MmInt {  // a compile-time int passed to a generic lambda
     static constexpr int value = N;
 };
 
-// ---- up to 32 tokens ------------------------------------------------------------
+// ---- few tokens ------------------------------------------------------------
 
 // One workgroup per 16 output rows (of each matrix) and tile of 16 NB tokens;
 // its eight waves take every eighth 256-byte block of the rows each and their

@@ -674,7 +674,7 @@ __device__ __attribute__((always_inline)) inline void split_rows_merge(const flo
             O += reinterpret_cast<const floatx4 *>(regions + w * region_bytes)[col * OC + (c ^ (col % 8))] * wt;
         }
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        *reinterpret_cast<floatx4 *>(p.out + ((int64_t)tok * p.n_head + kvh * G + col / QB) * HD + 4 * c) = O * inv;
+        *reinterpret_cast<floatx4_a4 *>(p.out + ((int64_t)tok * p.n_head + kvh * G + col / QB) * HD + 4 * c) = O * inv;
     }
 }
 
