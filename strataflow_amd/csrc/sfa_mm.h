@@ -170,17 +170,23 @@ __device__ inline half8 mm_half8(const floatx4 a, const floatx4 b) {
     return h;
 }
 
-// One step of Kahan's compensated sum: `sum` takes `v`, `comp` keeps what the
-// addition rounded away.  A product over thousands of k as one chain of
-// matrix-core additions is off by three to seven times what the one-token
-// kernels' 64 short lane sums are (k = 4096: 2.9e-7 against 0.9e-7 in f16,
-// 8.1e-7 against 1.2e-7 in f32), so the chains are cut at kMmChain additions or less
-// and their results summed this way.
+// Sums.  A product over thousands of k as one chain of matrix-core additions is
+// off by three to seven times what the one-token kernels' 64 short lane sums
+// are (k = 4096: 2.9e-7 against 0.9e-7 in f16, 8.1e-7 against 1.2e-7 in f32), so
+// both kernels keep short chains.  mm_skinny_kernel adds a 256-byte block's four
+// chains pairwise and the blocks of a wave with Kahan's compensated sum
+// (mm_kahan); mm_tile_kernel, where that costs 30 % of the time, adds in three
+// plain levels of at most kMmChain matrix-core or vector additions.
 constexpr int kMmChain = 8;
+
+// One step of the compensated sum: `sum` takes `v`, `comp` keeps what the
+// addition rounded away.  An infinite or NaN sum has no correction: its
+// (t - sum) - y would make NaN of an infinite sum at the next step.
 template <typename V>
 __device__ inline void mm_kahan(V &sum, V &comp, const V &v) {
-    const V y = v - comp, t = sum + y;
-    comp = (t - sum) - y;
+    const V y = v - comp, t = sum + y, c = (t - sum) - y;
+#pragma unroll
+    for (int j = 0; j < (int)(sizeof(V) / sizeof(float)); ++j) comp[j] = __builtin_isfinite(t[j]) ? c[j] : 0.0f;
     sum = t;
 }
 

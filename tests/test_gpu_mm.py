@@ -139,6 +139,71 @@ def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
         assert torch.equal(inplace, y)
 
 
+@pytest.mark.parametrize("n_rows", [1, 2, 3, 16, 17, 32, 33, 130])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_infinite_products(gpu, dtype, n_rows):
+    """One infinite product in a row's first, a middle or its last k block makes
+    that row's result infinite with the weight's sign, whatever is added before
+    and after it, and leaves the other rows' bits alone: an infinite activation,
+    one beyond f16's range beside F16 weights, an f32 product and an f32 sum that
+    overflow."""
+    from strataflow_amd import layer
+    n_in, n_out = 4096, 516
+    g = _gen(n_rows)
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    x = _rand(g, n_rows, n_in)
+    y, t = layer.mul_mat_vec(w, x), n_rows // 2
+    keep = [r for r in range(n_rows) if r != t]
+    assert torch.isfinite(y).all()
+    for col in (5, 300, 2050, n_in - 1):
+        wi = w.clone()
+        wi[:, col] = torch.where(wi[:, col] < 0, -2.0, 2.0).to(dtype)
+        base = layer.mul_mat_vec(wi, x)
+        for value in [float("inf"), -float("inf"), 70000.0 if dtype == torch.float16 else 3e38]:
+            xi = x.clone()
+            xi[t, col] = value
+            got = layer.mul_mat_vec(wi, xi)
+            assert torch.equal(got[t], torch.sign(wi[:, col].float()) * np.sign(value) * float("inf")), (col, value)
+            assert torch.equal(got[keep], base[keep])
+    if dtype == torch.float32:  # terms of one sign whose sum passes f32's range, block after block
+        wi, xi = torch.ones_like(w), x.clone()
+        xi[t] = 1e35
+        got = layer.mul_mat_vec(wi, xi)
+        assert torch.equal(got[t], torch.full_like(got[t], float("inf")))
+        assert torch.equal(got[keep], layer.mul_mat_vec(wi, x)[keep])
+
+
+@pytest.mark.parametrize("n_rows", [1, 2, 3, 13, 40, 150, 200])
+def test_infinite_expert_activations(gpu, n_rows):
+    """An activation beyond f16's range, in the first, a middle and the last k
+    block of the down product, in tokens routed to that expert: infinite with
+    the sign of the down weight, the other tokens' bits alone."""
+    from strataflow_amd import layer
+    n_embd, n_ff, n_expert, k = 256, 2304, 4, 2
+    g = _gen(n_rows)
+    h = torch.float16
+    gate, up = (_rand(g, n_expert, n_ff, n_embd, dtype=h, std=n_embd ** -0.5) for _ in range(2))
+    down = _rand(g, n_expert, n_embd, n_ff, dtype=h, std=n_ff ** -0.5)
+    x, res = _rand(g, n_rows, n_embd), _rand(g, n_rows, n_embd)
+    x[:, 0] = 1.0
+    wts = torch.full((n_rows, k), 0.5, device="cuda")
+    ids = torch.rand((n_rows, n_expert), generator=g, device="cuda").argsort(-1)[:, :k].int().contiguous()
+    ids[0] = torch.tensor([2, 0], device="cuda")
+    y = layer.moe_ffn(x, res, ids, wts, gate, up, down)
+    assert torch.isfinite(y).all()
+    hit = (ids == 2).any(1)
+    for col in (3, 1100, n_ff - 1):
+        gi, ui = gate.clone(), up.clone()
+        gi[2, col] = 0
+        ui[2, col] = 0
+        gi[2, col, 0] = ui[2, col, 0] = 400.0  # silu(400) * 400 = 160000
+        got = layer.moe_ffn(x, res, ids, wts, gi, ui, down)
+        want = (torch.sign(down[2, :, col].float()) * float("inf")).expand(int(hit.sum()), -1)
+        ok = down[2, :, col] != 0
+        assert torch.equal(got[hit][:, ok], want[:, ok]), col
+        assert torch.equal(got[~hit], y[~hit])
+
+
 def test_several_tokens_in_a_graph(gpu):
     """The calls replay from a captured graph with the bits of eager calls."""
     from strataflow_amd import layer
