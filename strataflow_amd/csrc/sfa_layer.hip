@@ -741,11 +741,11 @@ static bool mm_ok(int64_t n_rows, int64_t n_in, int64_t n_out, const void *w, co
            n_rows * n_in * 4 < ((int64_t)1 << 32) && aligned16(w) && aligned16(x);
 }
 
-template <typename WT, typename XT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
+template <typename WT, typename XT, bool SHORT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
 static void mm_tile_launch(const MmArgs<OUT> &p, int n_tiles, hipStream_t s) {
     constexpr int BMO = OUT == kMmGateUp ? BM / 2 : BM;
     const int n_rb8 = ((p.n_out + BMO - 1) / BMO + 7) / 8 * 8;
-    hipLaunchKernelGGL((mm_tile_kernel<WT, XT, BM, BN, WR, WC, KS, G, S, OUT>), dim3((unsigned)(n_rb8 * n_tiles)),
+    hipLaunchKernelGGL((mm_tile_kernel<WT, XT, SHORT, BM, BN, WR, WC, KS, G, S, OUT>), dim3((unsigned)(n_rb8 * n_tiles)),
                        dim3(64 * WR * WC * KS), 0, s, p);
 }
 
@@ -768,27 +768,36 @@ static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
     constexpr int kCus = 256;
     auto tiles = [&](int bm, int bn) { return (int64_t)((p.n_out + bm - 1) / bm) * ((n + bn - 1) / bn); };
     if constexpr (sizeof(WT) == 4) {
-        if (n <= 16)
-            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
-        else if (n <= 32)
-            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 2>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
-        else if (tiles(32, 32) <= 2 * kCus)
-            mm_tile_launch<WT, float, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+        auto launch = [&](auto sh) {
+            constexpr bool SHORT = decltype(sh)::value != 0;
+            if (n <= 16)
+                hipLaunchKernelGGL((mm_skinny_kernel<WT, float, SHORT, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+            else if (n <= 32)
+                hipLaunchKernelGGL((mm_skinny_kernel<WT, float, SHORT, OUT, 2>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+            else if (tiles(32, 32) <= 2 * kCus)
+                mm_tile_launch<WT, float, SHORT, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+            else if constexpr (SHORT)
+                mm_tile_launch<WT, float, true, 64, 64, 2, 2, 2, 1, 4>(p, (n + 63) / 64, s);
+            else
+                mm_tile_launch<WT, float, false, 64, 64, 2, 1, 4, 2, 2>(p, (n + 63) / 64, s);
+        };
+        if (p.n_in <= kMmShortF32)
+            launch(MmInt<1>{});
         else
-            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 2>(p, (n + 63) / 64, s);
+            launch(MmInt<0>{});
     } else {
         if (n <= 16 && p.n_out <= 16 * kCus)
-            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+            hipLaunchKernelGGL((mm_skinny_kernel<WT, float, false, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
         else if (tiles(32, 32) <= kCus)
-            mm_tile_launch<WT, float, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+            mm_tile_launch<WT, float, false, 32, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
         else if (tiles(64, 32) <= kCus)
-            mm_tile_launch<WT, float, 64, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
+            mm_tile_launch<WT, float, false, 64, 32, 1, 1, 4, 2, 4>(p, (n + 31) / 32, s);
         else if (tiles(64, 64) <= kCus)
-            mm_tile_launch<WT, float, 64, 64, 2, 1, 4, 2, 3>(p, (n + 63) / 64, s);
+            mm_tile_launch<WT, float, false, 64, 64, 2, 1, 4, 2, 3>(p, (n + 63) / 64, s);
         else if (tiles(128, 64) <= kCus)
-            mm_tile_launch<WT, float, 128, 64, 2, 2, 2, 1, 4>(p, (n + 63) / 64, s);
+            mm_tile_launch<WT, float, false, 128, 64, 2, 2, 2, 1, 4>(p, (n + 63) / 64, s);
         else
-            mm_tile_launch<WT, float, 128, 128, 2, 2, 2, 1, 3>(p, (n + 127) / 128, s);
+            mm_tile_launch<WT, float, false, 128, 128, 2, 2, 2, 1, 3>(p, (n + 127) / 128, s);
     }
 }
 
@@ -852,19 +861,19 @@ static bool moe_mm(const float *x, const float *residual, const int32_t *ids, co
     d.n_used = n_used;
     d.y = part;
     if (tile == 16) {
-        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, kMmGateUp, 1>), dim3((n_ff + 15) / 16, max_tiles),
+        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, false, kMmGateUp, 1>), dim3((n_ff + 15) / 16, max_tiles),
                            dim3(512), 0, s, g);
-        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, kMmDown, 1>), dim3((n_embd + 15) / 16, max_tiles),
+        hipLaunchKernelGGL((mm_skinny_kernel<_Float16, _Float16, false, kMmDown, 1>), dim3((n_embd + 15) / 16, max_tiles),
                            dim3(512), 0, s, d);
     } else if (tile == 64) {
-        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 4>(g, max_tiles, s);
-        mm_tile_launch<_Float16, _Float16, 128, 64, 2, 2, 2, 1, 4>(d, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 128, 64, 2, 2, 2, 1, 4>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 128, 64, 2, 2, 2, 1, 4>(d, max_tiles, s);
     } else if (mean <= 90) {
-        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 4>(g, max_tiles, s);
-        mm_tile_launch<_Float16, _Float16, 128, 128, 4, 2, 1, 1, 4>(d, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 128, 128, 4, 2, 1, 1, 4>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 128, 128, 4, 2, 1, 1, 4>(d, max_tiles, s);
     } else {
-        mm_tile_launch<_Float16, _Float16, 256, 128, 4, 2, 1, 1, 3>(g, max_tiles, s);
-        mm_tile_launch<_Float16, _Float16, 256, 128, 4, 2, 1, 1, 3>(d, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 256, 128, 4, 2, 1, 1, 3>(g, max_tiles, s);
+        mm_tile_launch<_Float16, _Float16, false, 256, 128, 4, 2, 1, 1, 3>(d, max_tiles, s);
     }
     hipLaunchKernelGGL(moe_combine_kernel, dim3((n_embd + 1023) / 1024, n_rows), dim3(256), 0, s, part, ids, weights,
                        residual, y, n_embd, n_expert, n_used);

@@ -177,7 +177,16 @@ __device__ inline half8 mm_half8(const floatx4 a, const floatx4 b) {
 // chains pairwise and the blocks of a wave with Kahan's compensated sum
 // (mm_kahan); mm_tile_kernel, where that costs 30 % of the time, adds in three
 // plain levels of at most kMmChain matrix-core or vector additions.
+// F32 rows of kMmShortF32 values or fewer (SHORT) need shorter chains than
+// that: the one-token kernels' chains of eight products meet in a tree.  There
+// a chain is four products and the chains meet in pairs.  Error against 64 bits
+// at 256 / 512 / 1024 values, in units of 1e-7: one token 0.81 / 0.86 / 0.99, few
+// tokens 0.92 / 0.96 / 0.99 without this and 0.78 / 0.83 / 0.87 with it, 32 x 32
+// tiles 0.87 / 0.91 / 0.96 and 0.79 / 0.84 / 0.89, 64 x 64 tiles 0.87 / 0.91 / 0.96
+// and 0.79 / 0.85 / 0.93.  Longer rows do without: the additions cost 3-16 % of
+// the time (4096 x 4096: 3 tokens 17.2 -> 18.2 us, 64 tokens 34.7 -> 40.2).
 constexpr int kMmChain = 8;
+constexpr int kMmShortF32 = 1024;
 
 // One step of the compensated sum: `sum` takes `v`, `comp` keeps what the
 // addition rounded away.  An infinite or NaN sum has no correction: its
@@ -204,7 +213,7 @@ struct MmInt {  // a compile-time int passed to a generic lambda
 // of each 64 bytes): the weights are read once per tile and the loads of CB
 // blocks are issued before any is used.  n_in * sizeof(WT) is a multiple of
 // 256.  Grid (row blocks, tiles).
-template <typename WT, typename XT, int OUT, int NB>
+template <typename WT, typename XT, bool SHORT, int OUT, int NB>
 __global__ __launch_bounds__(512) void mm_skinny_kernel(MmArgs<OUT> p) {
     constexpr int NM = OUT == kMmGateUp ? 2 : 1;
     constexpr bool F16W = sizeof(WT) == 2;
@@ -264,7 +273,7 @@ __global__ __launch_bounds__(512) void mm_skinny_kernel(MmArgs<OUT> p) {
 #pragma unroll
                 for (int h = 0; h < XM; ++h)
                     xv[b][s][h] = *reinterpret_cast<const intx4 *>(xr[b] + XM * (off + 64 * s) + 16 * h);
-        floatx4 acc[4][NM][NB];  // a chain for each 64 bytes
+        floatx4 acc[4][NM][NB];  // a chain for each 64 bytes (SHORT: the sum of its four)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -287,9 +296,15 @@ __global__ __launch_bounds__(512) void mm_skinny_kernel(MmArgs<OUT> p) {
 #pragma unroll
                     for (int m = 0; m < NM; ++m) {
                         const floatx4 wf = __builtin_bit_cast(floatx4, wv[m][s]);
+                        [[maybe_unused]] floatx4 c[4];
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[s][m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j], xf[j], acc[s][m][b], 0, 0, 0);
+                        for (int j = 0; j < 4; ++j) {
+                            if constexpr (SHORT)
+                                c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j], xf[j], zero, 0, 0, 0);
+                            else
+                                acc[s][m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j], xf[j], acc[s][m][b], 0, 0, 0);
+                        }
+                        if constexpr (SHORT) acc[s][m][b] = (c[0] + c[1]) + (c[2] + c[3]);
                     }
                 }
             }
@@ -379,7 +394,7 @@ constexpr int mm_min_waves(int nw, int lds_bytes) {
 // tokens of 4096 x 4096 as 32 x 32).
 // 1-D grid: the token tiles of one row block follow each other on one XCD
 // (XCD = L % 8), which reads its weight rows from HBM once.
-template <typename WT, typename XT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
+template <typename WT, typename XT, bool SHORT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
 __global__ __launch_bounds__(64 * WR * WC * KS, mm_min_waves(WR * WC * KS, mm_lds_bytes<WT, XT>(BM, BN, KS, G, S)))
 void mm_tile_kernel(MmArgs<OUT> p) {
     constexpr bool F16W = sizeof(WT) == 2;
@@ -466,14 +481,16 @@ void mm_tile_kernel(MmArgs<OUT> p) {
         }
     };
 
-    // Sums in three levels: chains of kChain k steps in acc (an F32 step is four
-    // additions), kMmChain of those in part, those in sum.
+    // Sums in three levels: chains of kChain k steps in acc, kMmChain of those in
+    // part, those in sum.  An F32 k step is a chain of eight products; SHORT: two
+    // of four, a stage's two steps are added in acc and part takes kMmChain steps.
     constexpr int kU = 4 / KS;                         // k steps of a slice per wave
     constexpr int kSteps = G * kU;                     // .. of a stage
-    constexpr int kChain = !F16W ? 1 : KS == 1 ? kMmChain : kMmChain / 2;  // k steps per chain
+    constexpr int kChain = !F16W ? (SHORT ? 2 : 1) : KS == 1 ? kMmChain : kMmChain / 2;  // k steps per chain
     constexpr int kPer = kChain > kSteps ? kChain / kSteps : 1;  // stages per chain
     constexpr int kUn = S % kPer == 0 ? S : kPer % S == 0 ? kPer : S * kPer;  // stages unrolled: slot and chain are fixed in each
     static_assert(kChain % kSteps == 0 || kSteps % kChain == 0, "chains end with a stage or within it");
+    static_assert(!SHORT || (!F16W && kSteps == 2), "SHORT: F32 rows, two steps a stage");
     const floatx16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     floatx16 acc[FR][FC], part[FR][FC], sum[FR][FC];
@@ -550,12 +567,23 @@ void mm_tile_kernel(MmArgs<OUT> p) {
                                                                                    first ? zero : acc[i][j], 0, 0, 0);
                         } else {
                             const floatx4 xf = __builtin_bit_cast(floatx4, c.b[j][0]);
+                            [[maybe_unused]] floatx16 half[FR][2];
 #pragma unroll
                             for (int k = 0; k < 4; ++k)
 #pragma unroll
-                                for (int i = 0; i < FR; ++i)
-                                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                        __builtin_bit_cast(floatx4, c.a[i])[k], xf[k], first && k == 0 ? zero : acc[i][j], 0, 0, 0);
+                                for (int i = 0; i < FR; ++i) {
+                                    floatx16 &s = SHORT ? half[i][k / 2] : acc[i][j];
+                                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                        __builtin_bit_cast(floatx4, c.a[i])[k], xf[k],
+                                        (SHORT ? k % 2 == 0 : first && k == 0) ? zero : s, 0, 0, 0);
+                                }
+                            if constexpr (SHORT) {
+#pragma unroll
+                                for (int i = 0; i < FR; ++i) {
+                                    half[i][0] += half[i][1];
+                                    acc[i][j] = first ? half[i][0] : acc[i][j] + half[i][0];
+                                }
+                            }
                         }
                     }
                     const bool last = kSteps >= kChain ? gv % kChain == kChain - 1 : un % kPer == kPer - 1 && gv == kSteps - 1;
@@ -567,7 +595,7 @@ void mm_tile_kernel(MmArgs<OUT> p) {
                     }
                 }
                 if (kSteps >= kChain || un % kPer == kPer - 1) {
-                    chains += kSteps >= kChain ? kSteps / kChain : 1;
+                    chains += SHORT ? kSteps : kSteps >= kChain ? kSteps / kChain : 1;
                     if (chains >= kMmChain) {
                         chains = 0;
 #pragma unroll

@@ -139,6 +139,28 @@ def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
         assert torch.equal(inplace, y)
 
 
+@pytest.mark.parametrize("n_in", [128, 256, 384, 512, 768, 1024, 1152])
+@pytest.mark.parametrize("n_rows", [3, 17, 40, 300])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_error_is_the_one_token_kernels(gpu, dtype, n_rows, n_in):
+    """No further from 64 bits than the one-token call, short rows above all,
+    whose one-token sums are chains of eight products in a tree.  The root mean
+    squares are over 16384 values or more each: 0.6 % of noise, 3 % allowed."""
+    from strataflow_amd import layer
+    g = _gen(n_rows + n_in)
+    n_out = 4096
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    x = _rand(g, max(n_rows, 8), n_in)
+
+    def err(y, rows):
+        return float((y.double() - _operand(rows, w) @ w.double().t()).square().mean().sqrt())
+
+    several = torch.cat([layer.mul_mat_vec(w, x[i:i + n_rows]) for i in ((0, 3, 5) if n_rows == 3 else (0,))])
+    rows = torch.cat([x[i:i + n_rows] for i in ((0, 3, 5) if n_rows == 3 else (0,))])
+    ones = torch.cat([layer.mul_mat_vec(w, x[t:t + 1]) for t in range(8)])
+    assert err(several, rows) < 1.03 * err(ones, x[:8])
+
+
 @pytest.mark.parametrize("n_rows", [1, 2, 3, 16, 17, 32, 33, 130])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_infinite_products(gpu, dtype, n_rows):
