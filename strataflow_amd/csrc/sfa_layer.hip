@@ -729,16 +729,47 @@ static int gemv_launch(const GemvParams &p, bool f16, hipStream_t s) {
 
 static bool aligned16(const void *a) { return reinterpret_cast<uintptr_t>(a) % 16 == 0; }
 
-// The matrix-core kernels take whole 256-byte blocks of 16-byte aligned rows
-// and 32-bit offsets into x and into a tile of W; a product with 64 outputs
-// or fewer keeps gemv_kernel, whose arithmetic sfa_moe_gate's equals bit for
-// bit, and so do two tokens, which it serves in one read of the weights
-// (4096 x 6144 F16: 14.4 us against 16.2; three: 20.8 against 16.6).  The rule reads only what sfa_mul_mat_vec and sfa_qkv_rope_kv_append
-// have in common (the shape, w and x), so both take the same kernel and their
-// results stay equal.
-static bool mm_ok(int64_t n_rows, int64_t n_in, int64_t n_out, const void *w, const void *x) {
-    return n_rows >= 3 && n_out > 64 && n_out % 4 == 0 && n_in % 128 == 0 && n_in < (1 << 22) &&
-           n_rows * n_in * 4 < ((int64_t)1 << 32) && aligned16(w) && aligned16(x);
+// What the matrix-core kernels take: whole 256-byte blocks of 16-byte aligned
+// rows, and 32-bit offsets into x and into a tile of W.
+static bool mm_fits(int64_t n_rows, int64_t n_in, int64_t n_out, const void *w, const void *x) {
+    return n_out % 4 == 0 && n_in % 128 == 0 && n_in < (1 << 22) && n_rows * n_in * 4 < ((int64_t)1 << 32) &&
+           aligned16(w) && aligned16(x);
+}
+
+// Whether the dense and the Q/K/V product run on them.  64 outputs or fewer
+// keep gemv_kernel, whose arithmetic sfa_moe_gate's equals bit for bit, and so
+// do two tokens, which it serves in one read of the weights (4096 x 6144 F16:
+// 14.4 us against 16.2; three: 20.8 against 16.6).  So does a matrix of few
+// outputs: the matrix-core kernels have few workgroups there, each a serial walk
+// of the rows for 16 tokens' operands, where gemv_kernel has a wave per output
+// and two, four or eight tokens and finds the weights in the L2s, up to 14 MB or
+// so of them.  us (one-token / matrix-core kernels, GPU time), n_in x n_out:
+//   tokens             3           7           16          64         128
+//   F32 2048 x 2048   4.5 / 7.0   6.7 / 7.7 ' 11.1 / 9.3 ' 35.6 / 18 ' -
+//   F32 1024 x 1024   2.6 / 4.6   3.5 / 4.9   4.9 / 5.6 ' 11.5 / 5.8 ' -
+//   F32 4096 x 512    3.3 / 11    6.3 / 13    11 / 16     20 / 16 '   57 / 16 '
+//   F32 4096 x 128    3.3 / 11    6.1 / 13    11 / 16     11 / 16     14 / 16
+//   F16 2048 x 2048   4.1 / 5.0   6.3 / 5.7 ' 10.8 / 7.1 ' 36 / 7.5 ' -
+//   F16 4096 x 1024   4.2 / 8.0   6.2 / 9.3   10.4 / 12.3 33 / 12 '   65 / 13 '
+//   F16 8192 x 1024   9.7 / 14    18 / 17 '   33 / 23 '   71 / 23 '   -
+//   F16 4096 x 128    3.7 / 7.9   5.6 / 9.2   9.6 / 12    9.7 / 12    10.4 / 12
+// (' takes the matrix cores).  sfa_qkv_rope_kv_append's own one-token kernel reads the
+// weights again for every token, so the lines are drawn where both gain or are
+// level (F16 2048 x 1536, 4 tokens: 7.0 / 7.7).  The rule reads only what
+// sfa_mul_mat_vec and sfa_qkv_rope_kv_append have in common (the shape, w and
+// x), so both take the same kernel and their results stay equal.
+static bool mm_ok(int64_t n_rows, int64_t n_in, int64_t n_out, bool f16, const void *w, const void *x) {
+    if (n_rows < 3 || n_out <= 64 || !mm_fits(n_rows, n_in, n_out, w, x)) return false;
+    constexpr int64_t kMiB = 1 << 20;
+    const int64_t row = n_in * (f16 ? 2 : 4), wb = row * n_out;
+    bool few;
+    if (n_rows <= 4)
+        few = (n_out <= 1024 || (n_out <= 2048 && n_in >= 2048)) && (n_rows == 3 || wb <= 16 * kMiB);
+    else if (n_rows < 8)
+        few = n_out <= 512 || (n_out <= 1024 && n_in >= 1024 && (n_out <= 768 || wb <= 14 * kMiB));
+    else  // a router of many experts, the K or V product of a few sequences
+        few = n_out < n_in && row >= 4096 && n_rows * n_out <= 16384 && n_rows * n_in * 4 <= 3 * kMiB && wb <= 14 * kMiB;
+    return !few;
 }
 
 template <typename WT, typename XT, bool SHORT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>
@@ -762,6 +793,9 @@ static void mm_tile_launch(const MmArgs<OUT> &p, int n_tiles, hipStream_t s) {
 // F32 (4096 x 4096): the matrix cores' f32 rate binds sooner: skinny to 32
 // tokens (28, 32 x 32: 36), 32 x 32 while it has two workgroups a CU (128
 // tokens: 56, 64 x 64: 82), then 64 x 64 (512 tokens: 154, 32 x 32: 199).
+// Before those, skinny tiles of 16 tokens while they have no more than one
+// workgroup a CU (1024 x 1024: 33 tokens 5.7, 32 x 32: 10, one-token kernel 8.0;
+// 4096 x 1024: 64 tokens 16, 32 x 32: 35; 2048 x 2048: 32 tokens 9.3, in one tile 14).
 template <typename WT, int OUT>
 static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
     const int n = p.n_rows;
@@ -770,8 +804,9 @@ static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
     if constexpr (sizeof(WT) == 4) {
         auto launch = [&](auto sh) {
             constexpr bool SHORT = decltype(sh)::value != 0;
-            if (n <= 16)
-                hipLaunchKernelGGL((mm_skinny_kernel<WT, float, SHORT, OUT, 1>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
+            if (n <= 16 || tiles(16, 16) <= kCus)
+                hipLaunchKernelGGL((mm_skinny_kernel<WT, float, SHORT, OUT, 1>), dim3((p.n_out + 15) / 16, (n + 15) / 16),
+                                   dim3(512), 0, s, p);
             else if (n <= 32)
                 hipLaunchKernelGGL((mm_skinny_kernel<WT, float, SHORT, OUT, 2>), dim3((p.n_out + 15) / 16), dim3(512), 0, s, p);
             else if (tiles(32, 32) <= 2 * kCus)
@@ -821,8 +856,8 @@ static bool moe_mm(const float *x, const float *residual, const int32_t *ids, co
                    const void *up, const void *down, int n_rows, int n_embd, int n_ff, int n_expert, int n_used,
                    void *workspace, float *y, hipStream_t s) {
     const int64_t n_pairs = (int64_t)n_rows * n_used;
-    if (n_rows < 3 || n_expert > kPlanMaxExperts || !mm_ok(n_pairs, n_embd, n_ff, gate, x) ||
-        !mm_ok(n_pairs, n_ff, n_embd, down, workspace) || !aligned16(up))
+    if (n_rows < 3 || n_expert > kPlanMaxExperts || n_ff <= 64 || n_embd <= 64 || !mm_fits(n_pairs, n_embd, n_ff, gate, x) ||
+        !mm_fits(n_pairs, n_ff, n_embd, down, workspace) || !aligned16(up))
         return false;
     const int mean = (int)(n_pairs / n_expert);
     const int tile = mean <= 6 ? 16 : mean <= 45 ? 64 : 128;
@@ -909,7 +944,7 @@ SFA_API int sfa_mul_mat_vec(const void *w, int32_t w_type, const float *x, const
         if (!sfa::weight_type_ok(w_type) || n_in % 8 != 0) return SFA_ERR_UNSUPPORTED;
         if ((n_rows + 7) / 8 > 65535) return SFA_ERR_UNSUPPORTED;  // token blocks on grid y
         if (n_rows == 0) return SFA_OK;
-        if (sfa::mm_ok(n_rows, n_in, n_out, w, x)) {
+        if (sfa::mm_ok(n_rows, n_in, n_out, w_type == SFA_KV_F16, w, x)) {
             sfa::MmArgs<sfa::kMmDense> a{};
             a.w = w;
             a.x = x;
@@ -1035,7 +1070,7 @@ SFA_API int sfa_qkv_rope_kv_append(const sfa_kv_desc *kv, const void *w_qkv, int
         a.max_pages = max_pages;
         const dim3 grid((unsigned)(p.n_out / sfa::kLayerWaves), (unsigned)n_tok);
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        if (sfa::mm_ok(n_tok, n_embd, p.n_out, w_qkv, x)) {  // sfa_mul_mat_vec's rule: the results stay equal
+        if (sfa::mm_ok(n_tok, n_embd, p.n_out, w_type == SFA_KV_F16, w_qkv, x)) {  // sfa_mul_mat_vec's rule: the results stay equal
             sfa::MmArgs<sfa::kMmQkv> m{};
             m.w = w_qkv;
             m.x = x;

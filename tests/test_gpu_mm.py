@@ -69,7 +69,10 @@ def test_products(gpu, dtype, n_rows, n_in, n_out):
 @pytest.mark.parametrize("wdtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("kv_type", ["f16", "f32"])
 @pytest.mark.parametrize("n_tok,shape", [(2, (8, 4, 32, 256)), (3, (8, 4, 32, 256)), (16, (4, 2, 64, 384)), (40, (16, 4, 128, 512)),
-                                         (130, (8, 4, 32, 256)), (300, (32, 8, 128, 1024))])
+                                         (130, (8, 4, 32, 256)), (300, (32, 8, 128, 1024)),
+                                         # few outputs: the one-token kernels, and just past them
+                                         (4, (8, 4, 64, 2048)), (4, (16, 4, 128, 2048)), (7, (8, 4, 64, 1024)), (5, (16, 4, 128, 1024)),
+                                         (16, (4, 1, 128, 4096)), (32, (4, 2, 64, 2048)), (40, (4, 2, 64, 2048)), (50, (8, 4, 32, 512))])
 def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
     """Bit for bit, with skipped tokens and a page that is not there."""
     from strataflow_amd import layer, synth
@@ -159,6 +162,39 @@ def test_error_is_the_one_token_kernels(gpu, dtype, n_rows, n_in):
     rows = torch.cat([x[i:i + n_rows] for i in ((0, 3, 5) if n_rows == 3 else (0,))])
     ones = torch.cat([layer.mul_mat_vec(w, x[t:t + 1]) for t in range(8)])
     assert err(several, rows) < 1.03 * err(ones, x[:8])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n_rows,n_in,n_out", [
+    (3, 256, 1024), (3, 8192, 2048), (4, 2048, 2048), (4, 512, 512), (7, 256, 512), (7, 1024, 1024), (5, 14336, 768),
+    (8, 2048, 1024), (16, 2048, 1024), (17, 2048, 384), (64, 4096, 128), (128, 4096, 128), (40, 2048, 404)])
+def test_few_outputs_stay_with_the_one_token_kernel(gpu, dtype, n_rows, n_in, n_out):
+    """A matrix of few outputs, where that kernel is the faster one: the bits of
+    the one-token calls."""
+    from strataflow_amd import layer
+    g = _gen(n_rows + n_in + n_out)
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    x = _rand(g, n_rows, n_in)
+    y = layer.mul_mat_vec(w, x)
+    assert torch.equal(y, torch.cat([layer.mul_mat_vec(w, x[t:t + 1]) for t in range(n_rows)]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n_rows,n_in,n_out", [
+    (4, 256, 1028), (5, 512, 1024), (8, 1024, 1024), (17, 2048, 1024), (129, 4096, 128), (33, 1024, 1024), (48, 512, 640),
+    (64, 1024, 2048), (100, 128, 400), (31, 2048, 2052)])
+def test_past_few_outputs(gpu, dtype, n_rows, n_in, n_out):
+    """The other side of that rule, and the tiles of 16 tokens that F32 weights
+    take there, against float64."""
+    from strataflow_amd import layer
+    g = _gen(n_rows + n_in + n_out)
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    x, r = _rand(g, n_rows, n_in), _rand(g, n_rows, n_out)
+    y = layer.mul_mat_vec(w, x)
+    ref = _operand(x, w) @ w.double().t()
+    assert float((y.double() - ref).abs().max() / ref.square().mean().sqrt()) < 3e-6
+    assert float((y.double() - ref).norm() / ref.norm()) < 2e-7
+    assert torch.equal(layer.mul_mat_vec(w, x, residual=r), y + r)
 
 
 @pytest.mark.parametrize("n_rows", [1, 2, 3, 16, 17, 32, 33, 130])
