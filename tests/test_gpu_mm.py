@@ -72,7 +72,7 @@ def test_products(gpu, dtype, n_rows, n_in, n_out):
                                          (130, (8, 4, 32, 256)), (300, (32, 8, 128, 1024)),
                                          # few outputs: the one-token kernels, and just past them
                                          (4, (8, 4, 64, 2048)), (4, (16, 4, 128, 2048)), (7, (8, 4, 64, 1024)), (5, (16, 4, 128, 1024)),
-                                         (16, (4, 1, 128, 4096)), (32, (4, 2, 64, 2048)), (40, (4, 2, 64, 2048)), (50, (8, 4, 32, 512))])
+                                         (16, (4, 1, 128, 4096)), (32, (4, 2, 64, 2048)), (40, (4, 2, 64, 2048)), (50, (8, 4, 32, 512)), (3, (16, 8, 64, 512))])
 def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
     """Bit for bit, with skipped tokens and a page that is not there."""
     from strataflow_amd import layer, synth
@@ -182,7 +182,7 @@ def test_few_outputs_stay_with_the_one_token_kernel(gpu, dtype, n_rows, n_in, n_
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("n_rows,n_in,n_out", [
     (4, 256, 1028), (5, 512, 1024), (8, 1024, 1024), (17, 2048, 1024), (129, 4096, 128), (33, 1024, 1024), (48, 512, 640),
-    (64, 1024, 2048), (100, 128, 400), (31, 2048, 2052)])
+    (64, 1024, 2048), (100, 128, 400), (31, 2048, 2052), (3, 512, 1028), (3, 4096, 2052), (16, 4096, 1028)])
 def test_past_few_outputs(gpu, dtype, n_rows, n_in, n_out):
     """The other side of that rule, and the tiles of 16 tokens that F32 weights
     take there, against float64."""
@@ -206,7 +206,7 @@ def test_infinite_products(gpu, dtype, n_rows):
     one beyond f16's range beside F16 weights, an f32 product and an f32 sum that
     overflow."""
     from strataflow_amd import layer
-    n_in, n_out = 4096, 516
+    n_in, n_out = 4096, 2052  # past the one-token kernels' few outputs
     g = _gen(n_rows)
     w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
     x = _rand(g, n_rows, n_in)
