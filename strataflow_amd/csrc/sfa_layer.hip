@@ -23,6 +23,7 @@
 // 16-byte chunks, several chunks in flight per lane; activations (a few KB)
 // come from L2.  Weights are row-major [n_out][n_in] (ggml ne =
 // [n_in, n_out]); expert stacks are [n_expert][n_out][n_in].
+#include <cmath>
 #include <exception>
 
 #include "sfa_layer.h"
@@ -838,25 +839,47 @@ static void mm_launch(const MmArgs<OUT> &p, hipStream_t s) {
 
 // ---- experts of several tokens -------------------------------------------------------
 
-// The experts of three or more tokens with F16 weights: the (token, slot) pairs
+// Whether grouping pays: what the one-pair kernels read more than once has to be
+// worth the two launches more (5 us, 32 MB) and the rate at which the grouped
+// kernels read an expert's weights, 5.2 TB/s against 6.4 or, rows under 2048
+// values, 5.7.  The ids are on the device, so the experts touched are those of
+// tokens that choose n_used of n_expert evenly.  us of one pair at a time / grouped
+// (means over six draws of ids; ' goes grouped), n_embd x n_ff x experts (used):
+//   tokens                     3           4           6           13
+//   4096 x 14336 x 8 (2)     332 / 305 ' 432 / 316 ' 644 / 389 ' 1388 / 495 '
+//   2048 x 5632 x 16 (2)      66 / 81     84 / 102   122 / 126 '  256 / 193 '
+//   2048 x 5632 x 8 (2)       64 / 75     79 / 76 '  115 / 94 '   241 / 119 '
+//   2048 x 4352 x 64 (6)     147 / 171   196 / 218   287 / 291 '  607 / 443 '
+//   1024 x 4096 x 64 (8)     115 / 105   149 / 133 ' 213 / 170 '  444 / 240 '
+//   512 x 2048 x 128 (4)    18.6 / 32   22.7 / 35   32.0 / 43    68.0 / 67.3
+//   256 x 1024 x 8 (2)       6.5 / 12.2  7.1 / 12.5  8.2 / 12.8  12.5 / 12.9
+// Two tokens stay with one pair at a time (235 us against 261 at the first shape).
+static bool moe_pays(int n_rows, int n_embd, int n_ff, int n_expert, int n_used) {
+    if (n_rows < 3) return false;
+    const double pairs = (double)n_rows * n_used;
+    const double touched = n_expert * (1.0 - std::pow(1.0 - (double)n_used / n_expert, n_rows));
+    return (pairs - (n_embd < 2048 ? 1.1 : 1.23) * touched) * 6.0 * n_embd * n_ff > 32e6;
+}
+
+// The experts of several tokens with F16 weights: the (token, slot) pairs
 // grouped by expert, so that an expert's weights are read once for all its
 // tokens (once a tile) and not once a pair.  The activations take half of the
 // caller's workspace (halves), the down product's rows and the plan the other
-// half; shapes whose rows do not fit there (n_ff < 2 n_embd), more than 256
-// experts and unaligned operands keep the one-pair kernels, as do two tokens
-// (four pairs seldom share an expert: 235 us against 261).  Tiles by the mean
+// half; shapes whose rows and plan do not fit there (n_ff <= 2 n_embd), more than 256
+// experts and unaligned operands keep the one-pair kernels.  Tiles by the mean
 // number of pairs an expert has (us of two of eight 4096 x 14336 experts a
 // token): up to 6 the skinny kernel, bound by the weights (13 tokens: 445, with
 // 64-pair tiles 528; 32 tokens 556 against 513); to 45 tiles of 64 (180
 // tokens: 548, 128-pair tiles 567); above, tiles of 128 pairs by 128 rows (256
 // tokens: 578 against 657 with 64 pairs, 655 with 256 rows) and, from 90, by
 // 256 rows, whose waves feed each operand to four products (512 tokens: 745
-// against 835).
+// against 835).  Two of sixteen 2048 x 5632 experts are near the read of all of
+// them (1.1 GB, 220 us) through all of these: 24 tokens 220, 64 218, 128 220, 512 253.
 static bool moe_mm(const float *x, const float *residual, const int32_t *ids, const float *weights, const void *gate,
                    const void *up, const void *down, int n_rows, int n_embd, int n_ff, int n_expert, int n_used,
                    void *workspace, float *y, hipStream_t s) {
     const int64_t n_pairs = (int64_t)n_rows * n_used;
-    if (n_rows < 3 || n_expert > kPlanMaxExperts || n_ff <= 64 || n_embd <= 64 || !mm_fits(n_pairs, n_embd, n_ff, gate, x) ||
+    if (n_expert > kPlanMaxExperts || !moe_pays(n_rows, n_embd, n_ff, n_expert, n_used) || !mm_fits(n_pairs, n_embd, n_ff, gate, x) ||
         !mm_fits(n_pairs, n_ff, n_embd, down, workspace) || !aligned16(up))
         return false;
     const int mean = (int)(n_pairs / n_expert);

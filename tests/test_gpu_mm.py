@@ -101,7 +101,8 @@ def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
 @pytest.mark.parametrize("n_rows,n_embd,n_ff,n_expert,k", [
     (3, 128, 384, 4, 2), (13, 256, 1024, 8, 2), (25, 256, 640, 8, 2), (70, 128, 384, 4, 3), (110, 256, 1024, 5, 2), (200, 256, 1024, 5, 2),
     (400, 128, 512, 2, 2), (150, 128, 512, 4, 2), (300, 384, 1152, 3, 2),
-    (6, 256, 384, 8, 2), (9, 128, 384, 300, 2), (2, 128, 384, 4, 2)])  # no room for the rows; too many experts; two tokens
+    (6, 256, 384, 8, 2), (9, 128, 384, 300, 2), (2, 128, 384, 4, 2),  # no room for the rows; too many experts; two tokens
+    (3, 1024, 4096, 4, 2), (13, 512, 2048, 8, 2), (24, 256, 1024, 16, 4), (60, 256, 768, 2, 1), (26, 1024, 2304, 16, 1)])  # grouped, 16 pairs a tile
 def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
     """Against float64 and, with the same bits wherever it is run from, against
     the tokens one at a time; ids outside the stack add nothing, one expert
@@ -237,7 +238,7 @@ def test_infinite_expert_activations(gpu, n_rows):
     block of the down product, in tokens routed to that expert: infinite with
     the sign of the down weight, the other tokens' bits alone."""
     from strataflow_amd import layer
-    n_embd, n_ff, n_expert, k = 256, 2304, 4, 2
+    n_embd, n_ff, n_expert, k = 1024, 2560, 4, 2
     g = _gen(n_rows)
     h = torch.float16
     gate, up = (_rand(g, n_expert, n_ff, n_embd, dtype=h, std=n_embd ** -0.5) for _ in range(2))
@@ -260,6 +261,25 @@ def test_infinite_expert_activations(gpu, n_rows):
         ok = down[2, :, col] != 0
         assert torch.equal(got[hit][:, ok], want[:, ok]), col
         assert torch.equal(got[~hit], y[~hit])
+
+
+@pytest.mark.parametrize("n_rows,n_embd,n_ff,n_expert,k", [
+    (3, 256, 1024, 8, 2), (13, 256, 1024, 8, 2), (8, 128, 512, 128, 4), (6, 1024, 3072, 8, 1), (3, 512, 2048, 16, 2),
+    (4, 2048, 4224, 16, 2)])
+def test_experts_that_seldom_share_stay_ungrouped(gpu, n_rows, n_embd, n_ff, n_expert, k):
+    """Where grouping would cost more than the weights it reads once less: the
+    bits of the tokens one at a time."""
+    from strataflow_amd import layer
+    g = _gen(n_rows + n_ff)
+    h = torch.float16
+    gate, up = (_rand(g, n_expert, n_ff, n_embd, dtype=h, std=n_embd ** -0.5) for _ in range(2))
+    down = _rand(g, n_expert, n_embd, n_ff, dtype=h, std=n_ff ** -0.5)
+    x, res = _rand(g, n_rows, n_embd), _rand(g, n_rows, n_embd)
+    wts = torch.rand((n_rows, k), generator=g, device="cuda")
+    ids = torch.rand((n_rows, n_expert), generator=g, device="cuda").argsort(-1)[:, :k].int().contiguous()
+    y = layer.moe_ffn(x, res, ids, wts, gate, up, down)
+    rows = [layer.moe_ffn(x[t:t + 1], res[t:t + 1], ids[t:t + 1], wts[t:t + 1], gate, up, down) for t in range(n_rows)]
+    assert torch.equal(y, torch.cat(rows))
 
 
 def test_several_tokens_in_a_graph(gpu):
