@@ -938,6 +938,10 @@ __global__ __launch_bounds__(64 * kF32Waves) void prefill_f32_kernel(PrefillPara
         // rows before the window read as 0 for P V (their P is 0)
         for (int r = 0; pos0 + r < rows.lo && r < kSBN; ++r)
             if (lane < CPR) *reinterpret_cast<floatx4 *>(vt + r * RB + 16 * lane) = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        // other lanes of the wave read them, whose LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const uint8_t *vl = vt + (4 * hh) * RB + 4 * (n & 3);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {

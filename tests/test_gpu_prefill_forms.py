@@ -66,3 +66,35 @@ def test_forms_agree(gpu, kv_type, form):
         ref = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ vh
         got = whole.view(n_tok, hq, hd)[:, h].double()
         assert float((got - ref).norm() / ref.norm()) < tol, h
+
+
+@pytest.mark.parametrize("kv_type", ["f32", "q8_0"])
+@pytest.mark.parametrize("shape,past,n_tok,lo", [
+    ((8, 2, 128), 700, 40, 161), ((8, 8, 64), 700, 100, 95), ((16, 2, 128), 300, 33, 31), ((8, 8, 64), 40, 20, 33),
+    ((32, 8, 128), 2000, 64, 1987)])
+def test_rows_before_the_window_do_not_reach_the_result(gpu, kv_type, shape, past, n_tok, lo):
+    """K and V rows before a window that starts inside a tile may hold anything:
+    the bits are those of the call with zeros there.  (The F32 kernel clears such
+    V rows in LDS, for other lanes of the wave to read.)"""
+    from strataflow_amd import synth
+    from strataflow_amd.paged_kv import SFA_KV_F32, SFA_KV_Q8_0, PagedKV
+    hq, hkv, hd = shape
+    n, page = past + n_tok, 64
+    n_pages = -(-n // page) + 2
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + lo)
+    pt = torch.from_numpy(synth.page_tables(np.random.default_rng(n), [n], page, n_pages)).cuda()
+    k, v = (torch.randn((n, hkv, hd), generator=g, device="cuda") for _ in range(2))
+    q = torch.randn((n_tok, hq, hd), generator=g, device="cuda")
+    seq, pos = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.arange(n, dtype=torch.int32, device="cuda")
+    outs = []
+    for fill in (0.0, 3e4, float("nan")):
+        if kv_type == "q8_0" and fill != fill:
+            continue  # a block's quants have no NaN
+        kv = PagedKV(1, hq, hkv, hd, {"f32": SFA_KV_F32, "q8_0": SFA_KV_Q8_0}[kv_type], page, n_pages)
+        k[:lo], v[:lo] = fill, fill
+        kv.append(0, k, v, seq, pos, pt)
+        outs.append(kv.prefill(0, q, pt[0], past, kv_lo=lo))
+    assert torch.isfinite(outs[0]).all()
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
