@@ -72,7 +72,9 @@ def test_products(gpu, dtype, n_rows, n_in, n_out):
                                          (130, (8, 4, 32, 256)), (300, (32, 8, 128, 1024)),
                                          # few outputs: the one-token kernels, and just past them
                                          (4, (8, 4, 64, 2048)), (4, (16, 4, 128, 2048)), (7, (8, 4, 64, 1024)), (5, (16, 4, 128, 1024)),
-                                         (16, (4, 1, 128, 4096)), (32, (4, 2, 64, 2048)), (40, (4, 2, 64, 2048)), (50, (8, 4, 32, 512)), (3, (16, 8, 64, 512))])
+                                         (16, (4, 1, 128, 4096)), (32, (4, 2, 64, 2048)), (40, (4, 2, 64, 2048)), (50, (8, 4, 32, 512)), (3, (16, 8, 64, 512)),
+                                         # 6144 outputs: F16 tiles of 64 x 32, 64 x 64 and 128 x 128
+                                         (64, (32, 8, 128, 256)), (128, (32, 8, 128, 256)), (512, (32, 8, 128, 384))])
 def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
     """Bit for bit, with skipped tokens and a page that is not there."""
     from strataflow_amd import layer, synth
@@ -104,9 +106,9 @@ def test_qkv_equals_product_then_append(gpu, wdtype, kv_type, n_tok, shape):
     (6, 256, 384, 8, 2), (9, 128, 384, 300, 2), (2, 128, 384, 4, 2),  # no room for the rows; too many experts; two tokens
     (3, 1024, 4096, 4, 2), (13, 512, 2048, 8, 2), (24, 256, 1024, 16, 4), (60, 256, 768, 2, 1), (26, 1024, 2304, 16, 1)])  # grouped, 16 pairs a tile
 def test_experts(gpu, n_rows, n_embd, n_ff, n_expert, k):
-    """Against float64 and, with the same bits wherever it is run from, against
-    the tokens one at a time; ids outside the stack add nothing, one expert
-    may hold every pair, and the result may be written over the residual."""
+    """Against float64 and against the tokens one at a time, within 2e-4 of the
+    largest output; ids outside the stack add nothing, one expert may hold every
+    pair, and the result written over the residual has the same bits."""
     from strataflow_amd import layer
     g = _gen(n_rows + n_embd + n_ff)
     h = torch.float16
@@ -196,6 +198,25 @@ def test_past_few_outputs(gpu, dtype, n_rows, n_in, n_out):
     assert float((y.double() - ref).abs().max() / ref.square().mean().sqrt()) < 3e-6
     assert float((y.double() - ref).norm() / ref.norm()) < 2e-7
     assert torch.equal(layer.mul_mat_vec(w, x, residual=r), y + r)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rows_past_two_gibibytes(gpu, dtype):
+    """Activations of more than 2 GiB: the kernels' 32-bit offsets are unsigned.
+    (x lies 2 GiB into its buffer, so an offset taken as signed would read other
+    values of it, which the comparison shows.)"""
+    from strataflow_amd import layer
+    n_rows, n_in, n_out = 133000, 4096, 132
+    g = _gen(7)
+    w = _rand(g, n_out, n_in, dtype=dtype, std=n_in ** -0.5)
+    buf = torch.randn((1 << 29) + n_rows * n_in, generator=g, device="cuda")
+    x = buf[1 << 29:].view(n_rows, n_in)
+    y = layer.mul_mat_vec(w, x)
+    rows = torch.tensor([0, 1, 65535, 65536, 131071, 131072, 131073, 132000, n_rows - 1], device="cuda")
+    ref = _operand(x[rows], w) @ w.double().t()
+    assert float((y[rows].double() - ref).abs().max() / ref.square().mean().sqrt()) < 3e-6
+    some = layer.mul_mat_vec(w, x[-300:].contiguous())
+    assert float((y[-300:] - some).abs().max()) < 1e-5
 
 
 @pytest.mark.parametrize("n_rows", [1, 2, 3, 16, 17, 32, 33, 130])

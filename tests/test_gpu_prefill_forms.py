@@ -24,6 +24,13 @@ FORMS = [
     ((16, 4, 128), 2000, 577, 256, 0),    # the split, three waves' tiles short of a round
     ((8, 8, 64), 600, 100, 64, 500),      # a window of few tiles: one group
     ((8, 8, 64), 700, 100, 64, 280),      # the split, two tiles a wave
+    ((32, 8, 128), 0, 1024, 256, 0),      # two groups, nothing for the second one to attend in the first block
+    ((32, 8, 128), 0, 777, 64, 0),        # the same for Q8_0 (one group for F16)
+    ((16, 4, 128), 4500, 100, 64, 0),     # the split over more pages than the page-id window holds
+    ((8, 8, 64), 4700, 64, 64, 300),      # the same, from a window's start
+    ((32, 8, 128), 4200, 700, 64, 0),     # two groups over more pages than that
+    ((16, 4, 128), 100, 1600, 64, 500),   # two groups, a window that hides everything from the first blocks
+    ((8, 2, 128), 100, 1600, 256, 500),   # the split, the same
 ]
 
 
@@ -54,7 +61,7 @@ def test_forms_agree(gpu, kv_type, form):
     rel = float((whole.double() - parts.double()).norm() / parts.double().norm())
     assert rel < tol and float((whole - parts).abs().max()) < 20 * tol, rel
     if kv_type == "q8_0":
-        return  # the forms quantise Q alike; the sweep compares them with the oracle, which does too
+        return  # the forms quantise Q alike; test_q8_two_groups_vs_oracle and the sweep compare them with the oracle, which does too
     pos = torch.arange(n, device="cuda")
     hidden = (pos[None] > past + torch.arange(n_tok, device="cuda")[:, None]) | (pos[None] < lo)
     if past > 4 * page:
@@ -64,8 +71,23 @@ def test_forms_agree(gpu, kv_type, form):
         kh, vh = c(k[:, h // (hq // hkv)]).contiguous(), c(v[:, h // (hq // hkv)]).contiguous()
         s = (q[:, h].double() @ kh.t()) / hd ** 0.5
         ref = torch.softmax(s.masked_fill(hidden, -float("inf")), -1) @ vh
+        ref[hidden.all(1)] = 0.0  # nothing attended
         got = whole.view(n_tok, hq, hd)[:, h].double()
         assert float((got - ref).norm() / ref.norm()) < tol, h
+
+
+@pytest.mark.parametrize("past,n_tok,page", [(0, 777, 64), (700, 600, 256), (4300, 530, 64)])
+def test_q8_two_groups_vs_oracle(gpu, oracle_mod, past, n_tok, page):
+    """The Q8_0 kernel with two groups of waves (more than half the CUs), which
+    the sweep's sizes do not take."""
+    from tests.helpers import assert_close
+    from tests.test_gpu_prefill import build, run
+    host, dev, pt, q, n_kv = build(oracle_mod, gpu, Hq=32, Hkv=8, hd=128, n_cached=past, T=n_tok, page_size=page,
+                                   seed=past + n_tok, kv_type=8)
+    out = run(dev, gpu, pt, q, past)
+    ref = host.attention(q[None], 32, pt, np.array([n_kv], np.int32), np.array([0], np.int32), T=n_tok,
+                         mode=oracle_mod.GGML)[0].reshape(n_tok, -1)
+    assert_close(out, ref, what=f"past {past} T {n_tok} page {page}")
 
 
 @pytest.mark.parametrize("kv_type", ["f32", "q8_0"])
