@@ -228,7 +228,11 @@ SFA_API int sfa_attn_decode_noalloc(const sfa_kv_desc *kv, const float *q, float
  * out: [T][n_head * head_dim] f32.  F32, F16 and Q8_0 caches (Q8_0 with
  * head_dim >= 64, as in decode).  The 64-position K/V tiles must each lie in
  * one page: page_size must be a multiple of 64 (SFA_ERR_UNSUPPORTED
- * otherwise). */
+ * otherwise).  The positions are cut over waves by the length of the chunk and
+ * of its span, and F16 and Q8_0 caches round a probability to f16 against the
+ * running maximum of its part: a token's output depends on the chunk it comes
+ * in within that rounding (2^-11 of a probability; F32 caches: the order of f32
+ * sums). */
 SFA_API int sfa_attn_prefill(const sfa_kv_desc *kv, const float *q, float *out,
                              const int32_t *page_table, int32_t max_pages,
                              int32_t q_pos0, int32_t T, int32_t kv_lo,

@@ -50,7 +50,12 @@ SFA_API int sfa_rms_norm(const float *x, const float *weight, float *y, int32_t 
  * (engine.cpp:1883-1885, 1912) and, with a residual, the wo projection plus
  * ggml_add (engine.cpp:1905-1906).  W [n_out][n_in] f32 or f16 (w_type);
  * n_in must be a multiple of 8 (SFA_ERR_UNSUPPORTED otherwise).  residual may
- * be null or alias y. */
+ * be null or alias y.
+ * Three or more tokens share a read of the weights on the matrix cores if n_in
+ * is a multiple of 128, n_out a multiple of 4 above 64 and w and x are 16-byte
+ * aligned; otherwise, and where n_out is small, up to eight tokens share one
+ * in the one-token kernel.  The products are the same; the order in which they
+ * are summed, and so a row's last bits, depends on n_rows and on the shape. */
 SFA_API int sfa_mul_mat_vec(const void *w, int32_t w_type, const float *x, const float *residual,
                             float *y, int32_t n_rows, int32_t n_in, int32_t n_out, void *stream);
 
@@ -90,15 +95,19 @@ SFA_API int sfa_moe_norm_gate(const float *x, const float *norm_weight, float ep
  *           token with seq or pos < 0, whose K/V are not written)
  *   seq, pos, page_table, max_pages, freq_base : as sfa_rope_kv_append.
  * F16 and F32 caches; SFA_ERR_UNSUPPORTED for Q8_0 (a block spans 16 RoPE
- * pairs: use the two calls) and for n_tok > 65535.  One or two tokens read the
- * weights once each; more share a read. */
+ * pairs: use the two calls) and for n_tok > 65535.  Where sfa_mul_mat_vec runs
+ * on the matrix cores (three or more tokens, n_embd a multiple of 128, w_qkv
+ * and x 16-byte aligned, not few outputs) this call does and shares a read of
+ * the weights; everywhere else it reads them once per token, and a long chunk
+ * is better served by the two calls. */
 SFA_API int sfa_qkv_rope_kv_append(const sfa_kv_desc *kv, const void *w_qkv, int32_t w_type,
                                    const float *x, int32_t n_embd, float *q, const int32_t *seq,
                                    const int32_t *pos, int32_t n_tok, const int32_t *page_table,
                                    int32_t max_pages, float freq_base, void *stream);
 
-/* Workspace bytes of sfa_moe_ffn (the SwiGLU activations, n_rows * n_used *
- * n_ff floats); 0 for an invalid shape. */
+/* Workspace bytes of sfa_moe_ffn: n_rows * n_used * n_ff floats, for the SwiGLU
+ * activations or, where the pairs are grouped by expert, the activations and x
+ * in f16, the down product's rows and the grouping; 0 for an invalid shape. */
 SFA_API size_t sfa_moe_workspace_bytes(int32_t n_rows, int32_t n_used, int32_t n_ff);
 
 /* The expert segment (build_expert_segment, engine.cpp:1964-1984): for each
@@ -109,7 +118,14 @@ SFA_API size_t sfa_moe_workspace_bytes(int32_t n_rows, int32_t n_used, int32_t n
  * all of w_type; n_embd and n_ff multiples of 8, n_used <= 8 (else
  * SFA_ERR_UNSUPPORTED).  An id outside
  * [0, n_expert) contributes nothing.  y must not alias x; it may alias
- * residual. */
+ * residual.
+ * Three or more tokens whose pairs share enough weights are grouped by expert,
+ * so that an expert is read once for all its tokens: F16 weights, n_expert <=
+ * 256, n_embd and n_ff multiples of 128, n_ff > 2 n_embd (the grouped form's
+ * rows must fit the workspace), x, the weights and the workspace 16-byte
+ * aligned.  Everything else, F32 weights included, reads an expert once per
+ * (token, slot) pair at any n_rows.  Which form runs depends on n_rows, and with it
+ * the order of the sums: a row's last bits do too. */
 SFA_API int sfa_moe_ffn(const float *x, const float *residual, const int32_t *ids,
                         const float *weights, const void *gate_exps, const void *up_exps,
                         const void *down_exps, int32_t w_type, int32_t n_rows, int32_t n_embd,

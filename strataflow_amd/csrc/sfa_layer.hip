@@ -17,8 +17,8 @@
 // scales by (float)(1/sum); sum_rows sums in double; the expert outputs are
 // multiplied by their weights, added in slot order, then the residual is added.
 //
-// Products of three or more tokens run on the matrix cores (sfa_mm.h).  The
-// kernels here are HBM-bound (one or two tokens per weight read):
+// Products of three or more tokens run on the matrix cores (sfa_mm.h) where
+// mm_ok and moe_pays say so.  The kernels here are HBM-bound at one or two tokens:
 // a wave owns one to four output rows and its lanes stream each row in
 // 16-byte chunks, several chunks in flight per lane; activations (a few KB)
 // come from L2.  Weights are row-major [n_out][n_in] (ggml ne =

@@ -5,14 +5,15 @@
 //
 // Two kernels share one description of the work (MmArgs) and one epilogue
 // (mm_emit):
-//   mm_skinny_kernel  few tokens (16; F32 weights 32): bound by the read of the
-//                     weights
+//   mm_skinny_kernel  tiles of 16 (F32 weights: or 32) tokens, where those are
+//                     few: bound by the read of the weights and its latency
 //   mm_tile_kernel    more tokens: 128-byte k slices of W and x through LDS
 // Both take the MFMA A operand from W (rows = outputs) and B from x (columns =
 // tokens), so a lane's accumulator holds four consecutive outputs of one
 // token.  Operands are those of the one-token kernels: F16 weights take the
 // activation rounded to f16 (RNE) and sum the products in f32, F32 weights
-// multiply and sum in f32; only the order of the sums differs.
+// multiply and sum in f32; only the order of the sums differs, so a token's
+// bits depend on how many it is multiplied with.
 #pragma once
 #include "sfa_append.h"
 
@@ -210,8 +211,8 @@ struct MmInt {  // a compile-time int passed to a generic lambda
 // its eight waves take every eighth 256-byte block of the rows each and their
 // partial sums meet in LDS, pair by pair.  The operands go straight from
 // memory to registers in MFMA order (lane = row l % 16, 16-byte piece l / 16
-// of each 64 bytes): the weights are read once per tile and the loads of CB
-// blocks are issued before any is used.  n_in * sizeof(WT) is a multiple of
+// of each 64 bytes): the weights are read once per tile and a block's loads
+// are issued before any is used.  n_in * sizeof(WT) is a multiple of
 // 256.  Grid (row blocks, tiles).
 template <typename WT, typename XT, bool SHORT, int OUT, int NB>
 __global__ __launch_bounds__(512) void mm_skinny_kernel(MmArgs<OUT> p) {
@@ -389,9 +390,9 @@ constexpr int mm_min_waves(int nw, int lds_bytes) {
 // groups' products meet in LDS, from where the epilogue stores whole rows.
 // The stage loop is unrolled over the ring, so that slots and chains are fixed
 // and a step's operands are read from LDS while the step before it multiplies:
-// read and used step by step, every product waited out an LDS read (moe of 512
-// tokens 58 % of the wave cycles waiting; 64 x 32 tiles 22 -> 17 us at 64
-// tokens of 4096 x 4096 as 32 x 32).
+// read and used step by step, every product waited out an LDS read (experts of
+// 512 tokens: waves waiting on counters 58 -> 42 % of their cycles, call 863 ->
+// 765 us; 4096 x 4096, 64 tokens, 32 x 32 tiles 22 -> 17 us).
 // 1-D grid: the token tiles of one row block follow each other on one XCD
 // (XCD = L % 8), which reads its weight rows from HBM once.
 template <typename WT, typename XT, bool SHORT, int BM, int BN, int WR, int WC, int KS, int G, int S, int OUT>

@@ -515,8 +515,8 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void prefill_f16_kernel(
         }
         l_run += ls;
 
-        // masking of S(t+1) only where it meets the window start, the
-        // diagonal or rows past T, or for an invalid page (wave-uniform)
+        // masking of S(t+1) only where it meets the window start or the
+        // diagonal, or for an invalid page (wave-uniform)
         if (t < tile1 && prefill_edge(rows, (t + KG) * kPBN, dead_next))
             prefill_mask(sn, rows, (t + KG) * kPBN, hh, dead_next);
         if constexpr (KG > 1) m_acc = m_run;  // O's and l's reference (the last S(t+1) is discarded)
@@ -554,8 +554,10 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void prefill_f16_kernel(
 // K(t + 8) is requested once S(t) has read K(t) and lands during the softmax
 // and P V; V(t + 8) once P V has read V(t), and lands during the next S and
 // softmax.  Two waves per SIMD fill each other's waits.  What bounds it is a
-// workgroup's own read of the history (4.2 MB of K and V in 48 us at 8100
-// positions, 90 GB/s a CU).
+// wave's chain per tile (load, S, softmax, P V), not the bytes: 93 tokens on
+// 8000 positions take 46 / 43 / 35 us at head_dim 128 / 64 / 32, 1.5 / 1.4 / 1.1 us
+// a tile of 16 / 8 / 4 KB (on busy CUs: matrix cores 30 % of the time, waves
+// waiting on counters 35 %, to issue 23 %, VALU 18 %).
 constexpr int kSplitWaves = 8;
 constexpr int kSBN = 32;  // positions per wave tile
 
@@ -1451,9 +1453,13 @@ __global__ __launch_bounds__(64 * kSplitWaves) void prefill_split_q8_kernel(Pref
 //   Q8_0  wg 200                 387 / 246 / 333     46 / 34 / 38
 //   Q8_0  wg 376                   - / 465 / 453      - / 57 / 70
 // So the split up to half the CUs and two groups up to all of them; short F16
-// spans above a quarter of the CUs stay with one group, and so do the shortest
-// of all, where nothing is gained (93 tokens alone: 10 us against 12) and one
-// group's rounding is what a short prompt's results have been.
+// spans above a quarter of the CUs stay with one group.  Spans under 512
+// positions do too, although the split is a few us faster there (256 tokens
+// alone: the first and fourth lines; 93 alone: 10 against 12): its probabilities
+// round to f16 against other running maxima, which moved an expert choice of the
+// tiny MoE model in one 95-token prompt of twenty, and short prompts keep the
+// results they had.  F32 caches always split; of 130 sizes measured the form
+// before it was faster at one (64 / 8 heads, 1024 tokens alone: 190 against 206).
 template <int HD, int G>
 static void launch_prefill(const PrefillParams &p, int kv_type, hipStream_t s) {
     constexpr int kCus = 256;
