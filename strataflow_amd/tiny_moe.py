@@ -263,6 +263,8 @@ class TinyMoeGpu(TinyMoe):
         dev = self.device
         ids_np = np.asarray(tokens, np.int64)
         T = ids_np.size
+        if isinstance(pos0, float):
+            pos0 = int(pos0)
         Hq, Hkv, hd = cfg.n_head, cfg.n_head_kv, cfg.head_dim
         if 0 <= pos0 and pos0 + T <= self.n_ctx:
             pos, seq, sl = self._pos[pos0:pos0 + T], self._zero[:T], self._pos[pos0 + T:pos0 + T + 1]

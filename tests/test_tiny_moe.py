@@ -78,3 +78,20 @@ def test_tiny_moe_whole_layer_on_gpu(gpu, oracle_mod, chunked):
           f"max per-step |dlogit|={dl:.3e} min top-2 margin={margin:.3e}")
     assert same, (ref[0], got[0])
     assert dl < 1e-3
+
+
+@pytest.mark.gpu
+def test_tiny_moe_positions_of_any_number_type(gpu):
+    """A position computed as a float, or by numpy or torch, is the same position,
+    for a prompt and for one token."""
+    import torch
+
+    from strataflow_amd.tiny_moe import TinyMoeGpu
+    cfg = TinyMoeConfig()
+    m = TinyMoeGpu(cfg, TinyMoeWeights(cfg, seed=0), 64, device=gpu)
+    toks = _prompt(cfg)
+    m.forward(toks[:8], 0)
+    for n in (1, 5):
+        want = m.forward(toks[8:8 + n], 8)
+        for pos0 in (8.0, np.float64(8), np.int64(8), torch.tensor(8)):
+            assert np.array_equal(m.forward(toks[8:8 + n], pos0), want)
